@@ -413,6 +413,363 @@ __global__ __launch_bounds__(kKqThreads) void kq_gemm_kernel(const uint8_t* __re
     }
 }
 
+// ---- Q4_K / Q6_K products of several activation rows, on the matrix cores ----------------
+// Per (output, super-block) the reference forms eight integer sums, one per
+// residue l = position mod 8, and chains each in fp32. A residue's sum is a
+// 32-term product: sum over (sub-block j, i) of (scale_j * q) * x. The scaled
+// weights are integers of at most 13 bits and x of 8, so fp16 operands hold
+// them exactly and every partial sum stays below 2^24: the fp32 accumulator of
+// an fp16 MFMA is the integer itself, already converted (32 * 4096 * 127 <
+// 2^24). Q4_K's scale * q <= 945 is one fp16; Q6_K's needs two, q = lo4 + 16
+// (hi2 - 2): lo4 * scale / 16 and (hi2 - 2) * scale, against x * 16.
+//
+// A workgroup owns 32 MT activation rows x 32 NT weight rows and wave l its
+// residue l: it decodes exactly the weights and activations of that residue
+// (nothing is decoded twice in a workgroup), multiplies them and runs the
+// outputs' sums[l] chains in its registers: acc += d * aux, super-blocks in
+// order. d = w.d * x.d comes as a 32 x 32 x 1 fp32 MFMA, one correctly rounded
+// product per output. Q4_K's mins term is a ninth sum over the sixteen sums of
+// 16 (|sum| <= 2032, exact in fp16), one tile on each of the first MT * NT
+// waves. At the end the waves' chains meet in shared memory and one lane per
+// output adds them in the reference's order. The raw blocks of the next
+// super-block are staged through shared memory (plane-major, so each wave
+// reads its residue's words) while the current one is multiplied.
+//
+// Bound: vector instructions. Per wave and super-block of a 64 x 64 tile 128
+// multiplies and adds run the chains; decoding, staging and addresses take ~230
+// more of the half-rate kinds (packed fp16, perm, and-or), the MFMAs (16 or 8
+// per wave, plus two fp32 ones that share the vector units) mostly run beside
+// them. Measured with the quantizer: Q6_K 512 rows x 4096, K 12288 2426 -> 198
+// us, Q4_K 509 rows x 4096, K 4096 410 -> 63 us (before: 4-way integer dots,
+// one lane per super-block and row, one chain lane per output).
+using h2_t = _Float16 __attribute__((ext_vector_type(2)));
+using h8_t = _Float16 __attribute__((ext_vector_type(8)));
+using f16v_t = float __attribute__((ext_vector_type(16)));
+using f32v_t = float __attribute__((ext_vector_type(32)));
+
+__device__ __forceinline__ h2_t as_h2(uint32_t v) { return __builtin_bit_cast(h2_t, v); }
+__device__ __forceinline__ uint32_t as_u32(h2_t v) { return __builtin_bit_cast(uint32_t, v); }
+__device__ __forceinline__ h2_t h2_fma(h2_t a, h2_t b, h2_t c) { return __builtin_elementwise_fma(a, b, c); }
+__device__ __forceinline__ h2_t h2_of(float v) { return h2_t{_Float16(v), _Float16(v)}; }
+__device__ __forceinline__ h8_t h8_of(h2_t a, h2_t b, h2_t c, h2_t d) {
+    const uint4 v = make_uint4(as_u32(a), as_u32(b), as_u32(c), as_u32(d));
+    return __builtin_bit_cast(h8_t, v);
+}
+// 1024 + byte, as fp16, of bytes 0 and 2 (even) or 1 and 3 (odd) of a dword
+__device__ __forceinline__ h2_t bytes_even(uint32_t v) { return as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04020400u)); }
+__device__ __forceinline__ h2_t bytes_odd(uint32_t v) { return as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04030401u)); }
+// 1024 + byte e of a dword, in both halves
+__device__ __forceinline__ h2_t byte_twice(uint32_t v, int e) { return as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04000400u | uint32_t(e) * 0x00010001u)); }
+
+constexpr int kMmThreads = 512;  // eight waves, one per residue
+// Up to this many rows kq_gemm_kernel is faster: it reads the weights with the
+// whole chip, where 32-row tiles leave N / 32 workgroups (4096 x 4096, 8 rows:
+// Q4_K 14.9 against 19.8 us, Q6_K 18.2 and 19.4; 16 rows: 23.1 and 19.8, 30.5 and 19.6).
+constexpr int kMmMinRows = 8;
+__device__ __forceinline__ uint32_t mm_chunk_index(uint32_t slot, int u, int U) { return ((slot / 64) * U + u) * 64 + slot % 64; }
+
+template <int TYPE, int MT, int NT>
+struct KqMmShared {
+    static constexpr int BM = 32 * MT, BN = 32 * NT;
+    static constexpr int U = TYPE == 12 ? 9 : 13;       // 16-byte chunks per weight block
+    static constexpr int XP = BM * 8 + 32;              // dwords per residue plane of x (padded: two planes' writes share no bank)
+    struct Stage {
+        uint32_t x[8 * XP];        // [residue][row][sub-block]: four int8, sign bit flipped
+        uint32_t w[4 * U * BN];    // [dword][row]
+        float xd[BM];
+        uint32_t bs[TYPE == 12 ? BM * 8 : 4];  // [row][16] fp16 sums of 16
+        float wd[BN];              // Q6_K
+    };
+    union {
+        Stage st[2];
+        float red[9 * 16 * 64];
+    };
+};
+
+template <int TYPE, int MT, int NT>
+__global__ __launch_bounds__(kMmThreads) void kq_mm_kernel(const uint8_t* __restrict__ w, const uint8_t* __restrict__ act, const uint32_t* __restrict__ xt,
+                                                           float* __restrict__ y, const float* __restrict__ resid, int64_t M, int64_t N, int K, int64_t ldy,
+                                                           int tiles_m, int tiles_n) {
+    using Sh = KqMmShared<TYPE, MT, NT>;
+    constexpr int BM = Sh::BM, BN = Sh::BN, U = Sh::U, XP = Sh::XP;
+    extern __shared__ __align__(16) uint8_t smem_mm[];
+    Sh& sh = *reinterpret_cast<Sh*>(smem_mm);
+    // workgroups go to the XCDs round robin: the row tiles of one weight tile
+    // take indices equal mod 8, so its weights are fetched into one L2
+    const int q8 = blockIdx.x / 8;
+    const int tn = (q8 / tiles_m) * 8 + blockIdx.x % 8, tm = q8 % tiles_m;
+    if (tn >= tiles_n) return;
+    const int tid = threadIdx.x, lane = tid & 63, l = __builtin_amdgcn_readfirstlane(tid >> 6), c32 = lane & 31, h = lane >> 5;
+    const int nb = K >> 8;
+    const int64_t m0 = int64_t(tm) * BM, n0 = int64_t(tn) * BN;
+    // Q4_K's 6-bit scales (mins) of sub-blocks 4h .. 4h + 3: h = 0 the low six
+    // bits of header dword 1 (2), h = 1 four bits of dword 3 under their top two
+    // a constant in a vector register: and-or of a mask and the fp16 1024 bits
+    // is then one instruction (its literal form takes two)
+    auto in_vgpr = [](uint32_t v) {
+        asm volatile("" : "+v"(v));
+        return v;
+    };
+    const uint32_t magic = 0x64006400u, lom = in_vgpr(0x000F000Fu), him = in_vgpr(0x00F000F0u);
+    uint32_t h2m[4];
+    if constexpr (TYPE == 14) {
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) h2m[jj] = in_vgpr(0x00030003u << (2 * jj));
+    }
+    const uint32_t hs2 = h ? 2u : 0u, hm6 = h ? 0x30303030u : 0x3F3F3F3Fu, hm4 = h ? 0x0F0F0F0Fu : 0u;
+
+    // ---- staging: this thread's chunks of a super-block
+    constexpr int XC = BM * 16, WC = BN * U;  // 16-byte chunks of x and of the weights
+    constexpr int XI = (XC + kMmThreads - 1) / kMmThreads, WI = (WC + kMmThreads - 1) / kMmThreads;
+    const int R = kq_rows_per_tile(K), wpt = kq_waves_per_tile(K);
+    // chunk indices fit 32 bits: the launcher checks
+    uint32_t xrow[XI];   // chunk tid % 16 of the row, super-block 0
+    uint32_t wslot[WI];  // slot of super-block 0 of the chunk's row
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+        const int idx = tid + i * kMmThreads;
+        xrow[i] = uint32_t(min<int64_t>(m0 + (idx / 16) % BM, M - 1) * nb * 16 + idx % 16);
+    }
+#pragma unroll
+    for (int i = 0; i < WI; ++i) {
+        const int64_t n = min<int64_t>(n0 + (tid + i * kMmThreads) % BN, N - 1);
+        wslot[i] = uint32_t(n / R * wpt * 64 + n % R);
+    }
+    const uint4* w4 = reinterpret_cast<const uint4*>(w);
+    const uint4* x4 = reinterpret_cast<const uint4*>(xt);
+    const uint16_t* dplane = reinterpret_cast<const uint16_t*>(w4 + kq_slots(N, K) * U);  // Q6_K
+    // threads 0 .. BM-1: a row's scale; BM .. 3 BM - 1 (Q4_K): half of a row's sums of 16; Q6_K: the last BN the weight scales
+    const int arow = tid < BM ? tid : (tid - BM) / 2;
+    const uint8_t* ablk = act + min<int64_t>(m0 + (arow % BM), M - 1) * nb * kQ8KBytes;
+    uint4 px[XI], pw[WI], pb;
+    float pd;
+    uint16_t ph;
+    auto load = [&](int b) {
+#pragma unroll
+        for (int i = 0; i < XI; ++i)
+            if (XC % kMmThreads == 0 || tid + i * kMmThreads < XC) px[i] = x4[xrow[i] + uint32_t(b) * 16];
+#pragma unroll
+        for (int i = 0; i < WI; ++i)
+            if (tid + i * kMmThreads < WC) pw[i] = w4[mm_chunk_index(wslot[i] + uint32_t(b * R), (tid + i * kMmThreads) / BN, U)];
+        if (tid < BM) {
+            pd = *reinterpret_cast<const float*>(ablk + int64_t(b) * kQ8KBytes);
+        } else if (TYPE == 12 && tid < 3 * BM) {
+            const uint32_t* s = reinterpret_cast<const uint32_t*>(ablk + int64_t(b) * kQ8KBytes + 260) + 4 * ((tid - BM) & 1);
+            pb = make_uint4(s[0], s[1], s[2], s[3]);
+        } else if (TYPE == 14 && tid >= kMmThreads - BN) {
+            ph = dplane[wslot[0] + uint32_t(b * R)];  // row tid % BN
+        }
+    };
+    auto store = [&](typename Sh::Stage& st) {
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            const int idx = tid + i * kMmThreads;
+            if (XC % kMmThreads == 0 || idx < XC) {
+                // chunk c of a row: sub-block c / 2, residues 4 (c % 2) .. + 3
+                uint32_t* dst = st.x + (4 * (idx & 1)) * XP + (idx / 16) * 8 + (idx % 16) / 2;
+                dst[0] = px[i].x ^ 0x80808080u;
+                dst[XP] = px[i].y ^ 0x80808080u;
+                dst[2 * XP] = px[i].z ^ 0x80808080u;
+                dst[3 * XP] = px[i].w ^ 0x80808080u;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < WI; ++i) {
+            const int idx = tid + i * kMmThreads;
+            if (idx < WC) {
+                uint32_t* dst = st.w + 4 * (idx / BN) * BN + idx % BN;
+                dst[0] = pw[i].x;
+                dst[BN] = pw[i].y;
+                dst[2 * BN] = pw[i].z;
+                dst[3 * BN] = pw[i].w;
+            }
+        }
+        if (tid < BM) {
+            st.xd[tid] = pd;
+        } else if (TYPE == 12 && tid < 3 * BM) {
+            auto two = [](uint32_t v) { return as_u32(h2_t{_Float16(int16_t(v & 0xFFFF)), _Float16(int16_t(v >> 16))}); };
+            reinterpret_cast<uint4*>(st.bs)[tid - BM] = make_uint4(two(pb.x), two(pb.y), two(pb.z), two(pb.w));
+        } else if (TYPE == 14 && tid >= kMmThreads - BN) {
+            st.wd[tid - (kMmThreads - BN)] = half_bits_to_f32(ph);
+        }
+    };
+
+    float acc[MT][NT][16], macc[16];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) macc[v] = 0.f;
+
+    load(0);
+    store(sh.st[0]);
+    if (nb > 1) load(1);
+    __syncthreads();
+    constexpr int F = TYPE == 12 ? 2 : 4;  // MFMA operands per 32 weight rows
+    // the weights of residue l, sub-blocks 4h .. 4h + 3, scaled
+    auto weights = [&](const typename Sh::Stage& st, int j, h8_t (&wf)[F], float& wd) {
+        const uint32_t* wr = st.w + 32 * j + c32;
+        if constexpr (TYPE == 12) {
+            wd = half_bits_to_f32(uint16_t(wr[0]));
+            const uint32_t h1 = wr[BN], h3 = wr[3 * BN];
+            const uint32_t sc = ((h1 >> hs2) & hm6) | (h3 & hm4);
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {  // sub-blocks 2c (low nibbles) and 2c + 1 of the four
+                const uint32_t g = wr[(4 + 8 * (2 * h + c) + l) * BN], g8 = g >> 8;
+                const h2_t s0 = byte_twice(sc, 2 * c) - h2_of(1024.f), s1 = (byte_twice(sc, 2 * c + 1) - h2_of(1024.f)) * h2_of(0.0625f);
+                const h2_t a0 = s0 * h2_of(-1024.f), a1 = s1 * h2_of(-1024.f);
+                // (1024 + q) s - 1024 s and (1024 + 16 q) s / 16 - 64 s: exact, one rounding each
+                wf[c] = h8_of(h2_fma(as_h2((g & lom) | magic), s0, a0), h2_fma(as_h2((g & him) | magic), s1, a1),
+                              h2_fma(as_h2((g8 & lom) | magic), s0, a0), h2_fma(as_h2((g8 & him) | magic), s1, a1));
+            }
+        } else {
+            wd = st.wd[32 * j + c32];
+            const uint32_t qh = wr[(32 + 8 * h + l) * BN], qh8 = qh >> 8;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {  // sub-blocks c (low nibbles) and c + 2 of the four
+                const uint32_t g = wr[(8 * (2 * h + c) + l) * BN], g8 = g >> 8;
+                h2_t lo[4], hi[4];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const int jj = c + 2 * t;
+                    // scales of the sub-block's halves (i = 0, 1 | 2, 3), int8
+                    const uint32_t sw = wr[(48 + 2 * h + jj / 2) * BN] ^ 0x80808080u;
+                    const h2_t s = as_h2(__builtin_amdgcn_perm(0x64646464u, sw, jj % 2 ? 0x04030402u : 0x04010400u)) - h2_of(1152.f);
+                    // low bits: lo4 s / 16 from 1024 + lo4 (or 1024 + 16 lo4)
+                    const h2_t ls = s * h2_of(t ? 0.00390625f : 0.0625f), la = s * h2_of(t ? -4.f : -64.f);
+                    const uint32_t lm = t ? him : lom;
+                    lo[t] = h2_fma(as_h2((g & lm) | magic), ls, la);
+                    lo[2 + t] = h2_fma(as_h2((g8 & lm) | magic), ls, la);
+                    // high bits, at 2 jj of each byte: (hi2 - 2) s
+                    const uint32_t hm = h2m[jj];
+                    const h2_t hs = s * h2_of(1.f / float(1 << (2 * jj))), hb = h2_of(-1024.f - float(2 << (2 * jj)));
+                    hi[t] = (as_h2((qh & hm) | magic) + hb) * hs;
+                    hi[2 + t] = (as_h2((qh8 & hm) | magic) + hb) * hs;
+                }
+                wf[2 * c] = h8_of(lo[0], lo[1], lo[2], lo[3]);
+                wf[2 * c + 1] = h8_of(hi[0], hi[1], hi[2], hi[3]);
+            }
+        }
+    };
+    // the activations of residue l, sub-blocks 4h .. 4h + 3 (Q6_K: times 16)
+    auto activations = [&](const typename Sh::Stage& st, h8_t (&xf)[MT][2], float& xd) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            const uint4 xv = *reinterpret_cast<const uint4*>(st.x + l * XP + (32 * i + c32) * 8 + 4 * h);
+            auto cv = [](h2_t t) {
+                if constexpr (TYPE == 12) return t - h2_of(1152.f);
+                return h2_fma(t, h2_of(16.f), h2_of(-18432.f));
+            };
+            const uint32_t a0 = xv.x, a1 = TYPE == 12 ? xv.y : xv.z, b0 = TYPE == 12 ? xv.z : xv.y, b1 = xv.w;
+            xf[i][0] = h8_of(cv(bytes_even(a0)), cv(bytes_even(a1)), cv(bytes_odd(a0)), cv(bytes_odd(a1)));
+            xf[i][1] = h8_of(cv(bytes_even(b0)), cv(bytes_even(b1)), cv(bytes_odd(b0)), cv(bytes_odd(b1)));
+        }
+        xd = st.xd[MT == 2 ? lane : c32];
+    };
+    auto products = [&](const h8_t (&xf)[MT][2], const h8_t (&wf)[F], f16v_t (&aux)[MT]) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            aux[i] = f16v_t{};
+#pragma unroll
+            for (int f = 0; f < F; ++f) aux[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[i][F == 2 ? f : f / 2], wf[f], aux[i], 0, 0, 0);
+        }
+    };
+    auto chains = [&](int j, float xd, float wd, const f16v_t (&aux)[MT]) {
+        const f32v_t d = __builtin_amdgcn_mfma_f32_32x32x1f32(xd, wd, f32v_t{}, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                acc[i][j][v] += d[16 * i + v] * aux[i][v];
+                asm volatile("" : "+v"(acc[i][j][v]));  // here, not sunk past what follows with d and aux kept
+            }
+        }
+    };
+    // One super-block's last chains run beside the next one's decoding, and its
+    // later products beside its first chains: the eight waves meet at a barrier
+    // per super-block, so what one wave does not overlap nothing does.
+    h8_t xf[MT][2], wf[F];
+    float xd, wd;
+    activations(sh.st[0], xf, xd);
+    weights(sh.st[0], 0, wf, wd);
+    for (int b = 0; b < nb; ++b) {
+        const auto& st = sh.st[b & 1];
+        const auto& nx = sh.st[(b + 1) & 1];
+        f16v_t aux[NT][MT];
+        // the other buffer's readers finished at the last barrier
+        if (b + 1 < nb) store(sh.st[(b + 1) & 1]);
+        if (b + 2 < nb) load(b + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (TYPE == 12) {
+            if (l < MT * NT) {  // the mins term of tile l
+                const int i = l % MT, j = l / MT;
+                const uint32_t* wr = st.w + 32 * j + c32;
+                const uint32_t h2 = wr[2 * BN], h3 = wr[3 * BN];
+                const float wdm = half_bits_to_f32(uint16_t(wr[0] >> 16)), xdm = st.xd[32 * i + c32];
+                const uint32_t mn = ((h2 >> hs2) & hm6) | ((h3 >> 4) & hm4);
+                const h8_t mf = h8_of(byte_twice(mn, 0) - h2_of(1024.f), byte_twice(mn, 1) - h2_of(1024.f), byte_twice(mn, 2) - h2_of(1024.f),
+                                      byte_twice(mn, 3) - h2_of(1024.f));
+                const h8_t bf = __builtin_bit_cast(h8_t, reinterpret_cast<const uint4*>(st.bs)[(32 * i + c32) * 2 + h]);
+                const f16v_t sumi = __builtin_amdgcn_mfma_f32_32x32x16_f16(bf, mf, f16v_t{}, 0, 0, 0);
+                // one product per output: the second of the two terms is 0 * 0
+                const f16v_t dm = __builtin_amdgcn_mfma_f32_32x32x2f32(h ? 0.f : xdm, h ? 0.f : wdm, f16v_t{}, 0, 0, 0);
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    macc[v] -= dm[v] * sumi[v];
+                    asm volatile("" : "+v"(macc[v]));
+                }
+            }
+        }
+        products(xf, wf, aux[0]);
+        if constexpr (NT == 2) {
+            h8_t wf1[F];
+            float wd1;
+            weights(st, 1, wf1, wd1);
+            __builtin_amdgcn_sched_barrier(0);
+            products(xf, wf1, aux[1]);
+            chains(0, xd, wd, aux[0]);
+            wd = wd1;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();
+        const float xdl = xd, wdl = wd;
+        activations(nx, xf, xd);  // past the last super-block: stale words, not used
+        weights(nx, 0, wf, wd);
+        chains(NT - 1, xdl, wdl, aux[NT - 1]);
+    }
+
+    // sumf = mins chain, then += sums[0..7]
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) sh.red[(l * 16 + v) * 64 + lane] = acc[i][j][v];
+            if (TYPE == 12 && l == j * MT + i) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) sh.red[(128 + v) * 64 + lane] = macc[v];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int e = tid; e < 1024; e += kMmThreads) {
+                float sumf = TYPE == 12 ? sh.red[8 * 1024 + e] : 0.f;
+#pragma unroll
+                for (int p = 0; p < 8; ++p) sumf += sh.red[p * 1024 + e];
+                const int v = e >> 6, el = e & 63;
+                const int64_t m = m0 + 32 * i + 8 * (v / 4) + 4 * (el >> 5) + v % 4, n = n0 + 32 * j + (el & 31);
+                if (m < M && n < N) {
+                    const int64_t o = m * ldy + n;
+                    y[o] = resid ? resid[o] + sumf : sumf;
+                }
+            }
+            __syncthreads();
+        }
+    }
+}
+
 // Q5_K against fp32 activations (no integer-activation kernel in the
 // reference): per block the dequant-in-dot chain of nm/src/quant.hpp:207-229
 // -- acc += (d1 * q - m1) * x, 256 products in order from acc = 0 -- and per
@@ -663,15 +1020,40 @@ static void kq_plan(int64_t M, int64_t N, int64_t K, int tile, int* R, int* rows
 
 int kquant_max_k(int type) { return type == 13 ? 16384 : 65536; }
 
+template <int TYPE, int MT, int NT>
+static void kq_mm(const uint8_t* w, const uint8_t* act, const uint32_t* xt, float* y, const float* resid, int64_t M, int64_t N, int64_t K, int64_t ldy,
+                  hipStream_t s) {
+    const int64_t tm = (M + 32 * MT - 1) / (32 * MT), tn = (N + 32 * NT - 1) / (32 * NT);
+    const dim3 grid(unsigned((tn + 7) / 8 * 8 * tm));
+    hipLaunchKernelGGL((kq_mm_kernel<TYPE, MT, NT>), grid, dim3(kMmThreads), sizeof(KqMmShared<TYPE, MT, NT>), s, w, act, xt, y, resid, M, N, int(K), ldy,
+                       int(tm), int(tn));
+}
+
 void launch_kquant_gemm_ld(int type, const void* w, const void* act, float* y, const float* resid, int64_t M, int64_t N, int64_t K, int64_t ldy,
                            hipStream_t s) {
-    int R, per;
-    kq_plan(M, N, K, kKqTile, &R, &per);
-    const dim3 grid(unsigned((N + R - 1) / R), unsigned((M + per - 1) / per));
     const int nb = int(K / 256);
     const auto* wb = static_cast<const uint8_t*>(w);
     const auto* ab = static_cast<const uint8_t*>(act);
     const uint32_t* xt = regrouped_of(act, M * nb);
+    if (M > kMmMinRows) {
+        // Rows go in slices whose chunk indices fit 32 bits. The small tile
+        // takes about half the large one's time per super-block (0.75 against
+        // 1.5 us) for a quarter of its outputs: whichever needs fewer rounds of
+        // one workgroup per compute unit, at those prices. Q4_K N 4096, K 4096:
+        // 64 rows 21 (small) and 33 us, 509 rows 98 and 63 us.
+        const int64_t slice = int64_t(1) << 20;
+        for (int64_t r0 = 0; r0 < M; r0 += slice) {
+            const int64_t rows = std::min(slice, M - r0);
+            const int64_t cus = device_cus();
+            const int64_t small = ((rows + 31) / 32 * ((N + 31) / 32) + cus - 1) / cus, large = ((rows + 63) / 64 * ((N + 63) / 64) + cus - 1) / cus;
+            auto run = small <= 2 * large ? (type == 12 ? kq_mm<12, 1, 1> : kq_mm<14, 1, 1>) : (type == 12 ? kq_mm<12, 2, 2> : kq_mm<14, 2, 2>);
+            run(wb, ab + r0 * nb * kQ8KBytes, xt + r0 * nb * 64, y + r0 * ldy, resid ? resid + r0 * ldy : nullptr, rows, N, K, ldy, s);
+        }
+        return;
+    }
+    int R, per;
+    kq_plan(M, N, K, kKqTile, &R, &per);
+    const dim3 grid(unsigned((N + R - 1) / R), unsigned((M + per - 1) / per));
     if (type == 12) {
         const size_t lds = size_t(kKqTile) * R * nb * 9 * 4;
         auto kernel = M == 1 ? kq_gemm_kernel<12, true> : kq_gemm_kernel<12, false>;
