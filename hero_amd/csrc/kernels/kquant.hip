@@ -885,6 +885,150 @@ __global__ __launch_bounds__(kKqThreads) void q5k_gemm_kernel(const uint8_t* __r
     }
 }
 
+// ---- Q5_K products of several activation rows ---------------------------------------------
+// The reference rounds each product wv * x and then each sum, 256 in order per
+// super-block, so nothing can be contracted; the work is one multiply and one
+// add per weight and row. The multiplies of a position's R rows x 64 weight
+// rows come as one fp32 MFMA of depth 1 (an outer product with a zero addend:
+// every entry the correctly rounded product), which needs one value of x and
+// one weight per lane where vector multiplies would need every row's x
+// broadcast to each lane; the adds are vector instructions. Lane n decodes the
+// weights of row n once for the R rows.
+//
+// A workgroup owns R activation rows x 64 weight rows; its eight waves take
+// super-blocks w, w + 8, ... each with its 256-term chains in registers, and
+// after every eight super-blocks one lane per output adds their results in
+// order. Each wave stages its own x, 64 positions at a time, in shared memory
+// (rows padded: 16 rows' 16-byte reads share no bank); no other wave reads it.
+//
+// Bound: the fp32 MFMA runs on the vector units, so a position of 16 rows costs
+// a SIMD 34 clocks of products, 36 of adds and ~15 of decoding. Measured: 256
+// rows x 4096, K 4096 506 -> 173 us, of which the multiplies and adds alone are
+// 134 (before: every lane decoding its block per 4 rows, x from shared memory).
+template <int R>
+struct OuterF32;
+template <>
+struct OuterF32<4> {
+    using V = float __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ V mul(float x, float w) { return __builtin_amdgcn_mfma_f32_4x4x1f32(x, w, V{}, 0, 0, 0); }
+    static __device__ __forceinline__ int row(int v, int) { return v; }
+    static __device__ __forceinline__ int col(int, int lane) { return lane; }
+};
+template <>
+struct OuterF32<16> {
+    using V = float __attribute__((ext_vector_type(16)));
+    static __device__ __forceinline__ V mul(float x, float w) { return __builtin_amdgcn_mfma_f32_16x16x1f32(x, w, V{}, 0, 0, 0); }
+    static __device__ __forceinline__ int row(int v, int lane) { return 4 * (lane >> 4) + (v & 3); }
+    static __device__ __forceinline__ int col(int v, int lane) { return 16 * (v >> 2) + (lane & 15); }
+};
+constexpr int kQ5Waves = 8;
+constexpr int kQ5Pos = 64;             // positions staged at a time
+constexpr int kQ5Ld = kQ5Pos + 4;      // padded row
+constexpr size_t q5k_mm_shared(int R) { return size_t(kQ5Waves) * R * kQ5Ld * 4; }
+
+template <int R>
+__global__ __launch_bounds__(64 * kQ5Waves) void q5k_mm_kernel(const uint8_t* __restrict__ w, const float* __restrict__ x, int64_t ldx, float* __restrict__ y,
+                                                               const float* __restrict__ resid, int64_t M, int64_t N, int K, int64_t ldy) {
+    using Outer = OuterF32<R>;
+    using V = typename Outer::V;
+    extern __shared__ __align__(16) float smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nb = K >> 8;
+    const int64_t n0 = int64_t(blockIdx.x) * 64, m0 = int64_t(blockIdx.y) * R;
+    float* xs = smem + wave * R * kQ5Ld;
+    const int64_t n = min<int64_t>(n0 + lane, N - 1);
+    const int rows_per_tile = kq_rows_per_tile(K);
+    const int64_t slot0 = n / rows_per_tile * kq_waves_per_tile(K) * 64 + n % rows_per_tile;
+
+    // staging of 64 positions of R rows: 16 lanes per row
+    constexpr int XI = R / 4;
+    const float* xrow[XI];
+#pragma unroll
+    for (int i = 0; i < XI; ++i) xrow[i] = x + min<int64_t>(m0 + 4 * i + lane / 16, M - 1) * ldx + 4 * (lane % 16);
+    float4 px[XI];
+    auto load = [&](int k) {
+#pragma unroll
+        for (int i = 0; i < XI; ++i) px[i] = *reinterpret_cast<const float4*>(xrow[i] + k);
+    };
+
+    constexpr int OUT = R * 64 / (64 * kQ5Waves) > 0 ? R * 64 / (64 * kQ5Waves) : 1;
+    float sum[OUT];
+#pragma unroll
+    for (int i = 0; i < OUT; ++i) sum[i] = 0.f;
+
+    for (int b0 = 0; b0 < nb; b0 += kQ5Waves) {
+        const int b = b0 + wave;
+        if (b < nb) {
+            load(256 * b);
+            const int64_t slot = slot0 + int64_t(b) * rows_per_tile;
+            const uint4* src = reinterpret_cast<const uint4*>(w) + kq_chunk_index(slot, 0, 11);  // chunk u at src[64 u]
+            const uint4 hdr = src[0], h0 = src[64], h1 = src[128];
+            // the 6-bit scales and mins of sub-blocks 0..3 and 4..7, a byte each
+            const uint32_t sc4[2] = {hdr.y & 0x3F3F3F3Fu, (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u)};
+            const uint32_t mn4[2] = {hdr.z & 0x3F3F3F3Fu, ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u)};
+            const float d = half_bits_to_f32(uint16_t(hdr.x & 0xFFFF)), dmin = half_bits_to_f32(uint16_t(hdr.x >> 16));
+            uint32_t qh[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
+            uint4 q0 = src[64 * 3], q1 = src[64 * 4];
+            V acc{}, prod{};  // prod: the products of the position before, added while the next ones form
+#pragma unroll 1
+            for (int c = 0; c < 4; ++c) {
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int i = 0; i < XI; ++i) *reinterpret_cast<float4*>(xs + (4 * i + lane / 16) * kQ5Ld + 4 * (lane % 16)) = px[i];
+                __builtin_amdgcn_wave_barrier();
+                const uint32_t qs[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+                if (c < 3) {
+                    load(256 * b + kQ5Pos * (c + 1));
+                    q0 = src[64 * (3 + 2 * (c + 1))], q1 = src[64 * (4 + 2 * (c + 1))];
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                const float* xl = xs + (lane % R) * kQ5Ld;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    const int j = 2 * c + h;
+                    const float d1 = d * float((sc4[c >> 1] >> (8 * (j & 3))) & 0xFFu), m1 = dmin * float((mn4[c >> 1] >> (8 * (j & 3))) & 0xFFu);
+#pragma unroll
+                    for (int i4 = 0; i4 < 8; ++i4) {
+                        const float4 xv = *reinterpret_cast<const float4*>(xl + 32 * h + 4 * i4);
+                        // byte u = the 4-bit value + 16 * its fifth bit (bit j of byte u of qh)
+                        const uint32_t q5 = ((qs[i4] >> (4 * h)) & 0x0F0F0F0Fu) | (((qh[i4] >> j) & 0x01010101u) << 4);
+                        const float xe[4] = {xv.x, xv.y, xv.z, xv.w};
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            const float wv = d1 * float((q5 >> (8 * u)) & 0xFFu) - m1;
+                            const V next = Outer::mul(xe[u], wv);
+                            acc += prod;
+                            prod = next;
+                            __builtin_amdgcn_sched_barrier(0);
+                        }
+                    }
+                }
+            }
+            acc += prod;
+            __builtin_amdgcn_wave_barrier();
+            float* res = xs;  // [R][64]
+#pragma unroll
+            for (int v = 0; v < R; ++v) res[Outer::row(v, lane) * 64 + Outer::col(v, lane)] = acc[v];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < OUT; ++i) {
+            const int e = tid + 64 * kQ5Waves * i;
+            if (e < R * 64)
+                for (int p = 0; p < min(kQ5Waves, nb - b0); ++p) sum[i] += smem[p * R * kQ5Ld + e];
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < OUT; ++i) {
+        const int e = tid + 64 * kQ5Waves * i;
+        const int64_t m = m0 + e / 64, nn = n0 + e % 64;
+        if (e < R * 64 && m < M && nn < N) {
+            const int64_t o = m * ldy + nn;
+            y[o] = resid ? resid[o] + sum[i] : sum[i];
+        }
+    }
+}
+
 // GGUF -> packed K-quant layout. Within a block: Q4_K keeps its 16-byte
 // header; its 128 quant bytes become 32 residue dwords: dword 8c + l, byte i =
 // qs[32c + 8i + l] (low nibbles: sub-block 2c, high: 2c + 1). Q6_K's 128 ql
@@ -1074,6 +1218,31 @@ void launch_q5k_gemm(const void* w, const float* x, int64_t ldx, float* y, const
     const int tile = M == 1 ? 1 : K <= 4096 ? 4 : K <= 8192 ? 2 : 1;
     int R, per;
     kq_plan(M, N, K, tile, &R, &per);
+    // Several rows: the matrix-core form unless the lane-per-block form's
+    // workgroup passes (one per R weight rows and tile activation rows; about 8,
+    // 6.6 and 5 us each on a compute unit, at least 13) cost less than its 4-row
+    // tiles (about 3 + 1.2 us per super-block of a row), both in microseconds.
+    // Measured, former and this form: K 4096 x 4096 rows: 8 rows 19.4 / 22.1 us,
+    // 10 rows 35.4 / 22.7; K 1024 x 1000, 2 rows: 12.8 / 9.4; K 8192 x 4096, 4
+    // rows 27.3 / 39.8, 8 rows 53.2 / 41.1; K 12288 x 4096, 2 rows 45 / 62, 4 rows 80 / 61.
+    if (M > 1) {
+        const int64_t cus = device_cus(), nb = K / 256;
+        auto rounds = [&](int64_t rows, int64_t cols) { return ((M + rows - 1) / rows * ((N + cols - 1) / cols) + cus - 1) / cus; };
+        const double lanes = std::max(13.0, double(rounds(tile, R)) * (tile == 4 ? 8.0 : tile == 2 ? 6.6 : 5.0));
+        if (double(rounds(4, 64)) * (3.0 + 1.2 * double(nb)) < lanes) {
+            // 16-row tiles take three times a 4-row tile's time once the compute
+            // units are full (47 and 15.5 us at K 4096)
+            const int rows = 3 * rounds(16, 64) < rounds(4, 64) ? 16 : 4;
+            const int64_t slice = int64_t(65535) * rows;  // grid.y
+            for (int64_t r0 = 0; r0 < M; r0 += slice) {
+                const int64_t part = std::min(slice, M - r0);
+                hipLaunchKernelGGL(rows == 16 ? q5k_mm_kernel<16> : q5k_mm_kernel<4>, dim3(unsigned((N + 63) / 64), unsigned((part + rows - 1) / rows)),
+                                   dim3(64 * kQ5Waves), q5k_mm_shared(rows), s, static_cast<const uint8_t*>(w), x + r0 * ldx, ldx, y + r0 * ldy,
+                                   resid ? resid + r0 * ldy : nullptr, part, N, int(K), ldy);
+            }
+            return;
+        }
+    }
     const dim3 grid(unsigned((N + R - 1) / R), unsigned((M + per - 1) / per));
     const size_t lds = size_t(tile) * K * 4;  // <= 64 KiB
     const auto* wb = static_cast<const uint8_t*>(w);

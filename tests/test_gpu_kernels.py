@@ -916,6 +916,21 @@ def test_q5_K_gemm_matches_oracle_bitwise(lib, m, n, k):
     assert bad.size == 0, f"{bad.size} outputs differ, first {bad[:5]}"
 
 
+# the outer-product form: edges of its 4- and 16-row tiles and 64-row weight
+# tiles, fewer super-blocks than waves, more than a round of them; the tiny
+# scales make products and sums subnormal. Products and sums are each rounded
+# once, in the reference's order: equal bit for bit.
+@pytest.mark.parametrize("m,n,k", [(2, 1, 256), (3, 65, 256), (5, 64, 1024), (10, 4097, 2304), (70, 800, 5120), (14, 2050, 8192), (250, 1020, 2304), (497, 511, 1280)])
+@pytest.mark.parametrize("scale", [1.0, 1e-36])
+def test_q5_K_outer_product_form_matches_oracle_bitwise(lib, m, n, k, scale):
+    rng = np.random.default_rng(m * 1009 + n * 31 + k)
+    w = q5k_weights(rng, n, k)
+    x = (rng.standard_normal((m, k)) * scale).astype(np.float32)
+    y = q5k_dev(lib, w, x, n, k)
+    expect = oracle.linear(oracle.Q5_K, w, n, k, x)
+    assert np.array_equal(bits(y), bits(expect))
+
+
 @pytest.mark.parametrize("wtype,name", [(12, "kq_w4"), (13, "kq_w5"), (14, "kq_w6")])
 def test_kquant_dequant_rows_match_reference_golden(lib, kernels_golden, wtype, name):
     """Weight::dequant_row of rows 0 and 37 (the embedding gather), the
