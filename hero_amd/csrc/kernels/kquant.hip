@@ -462,10 +462,6 @@ __device__ __forceinline__ h2_t bytes_odd(uint32_t v) { return as_h2(__builtin_a
 __device__ __forceinline__ h2_t byte_twice(uint32_t v, int e) { return as_h2(__builtin_amdgcn_perm(0x64646464u, v, 0x04000400u | uint32_t(e) * 0x00010001u)); }
 
 constexpr int kMmThreads = 512;  // eight waves, one per residue
-// Up to this many rows kq_gemm_kernel is faster: it reads the weights with the
-// whole chip, where 32-row tiles leave N / 32 workgroups (4096 x 4096, 8 rows:
-// Q4_K 14.9 against 19.8 us, Q6_K 18.2 and 19.4; 16 rows: 23.1 and 19.8, 30.5 and 19.6).
-constexpr int kMmMinRows = 8;
 __device__ __forceinline__ uint32_t mm_chunk_index(uint32_t slot, int u, int U) { return ((slot / 64) * U + u) * 64 + slot % 64; }
 
 template <int TYPE, int MT, int NT>
@@ -1179,21 +1175,31 @@ void launch_kquant_gemm_ld(int type, const void* w, const void* act, float* y, c
     const auto* wb = static_cast<const uint8_t*>(w);
     const auto* ab = static_cast<const uint8_t*>(act);
     const uint32_t* xt = regrouped_of(act, M * nb);
-    if (M > kMmMinRows) {
-        // Rows go in slices whose chunk indices fit 32 bits. The small tile
-        // takes about half the large one's time per super-block (0.75 against
-        // 1.5 us) for a quarter of its outputs: whichever needs fewer rounds of
-        // one workgroup per compute unit, at those prices. Q4_K N 4096, K 4096:
-        // 64 rows 21 (small) and 33 us, 509 rows 98 and 63 us.
-        const int64_t slice = int64_t(1) << 20;
-        for (int64_t r0 = 0; r0 < M; r0 += slice) {
-            const int64_t rows = std::min(slice, M - r0);
-            const int64_t cus = device_cus();
-            const int64_t small = ((rows + 31) / 32 * ((N + 31) / 32) + cus - 1) / cus, large = ((rows + 63) / 64 * ((N + 63) / 64) + cus - 1) / cus;
+    if (M > 1) {
+        // Which form, by estimates in microseconds (with the quantizer, fitted to
+        // M 2 .. 48, N 1000 .. 12288, K 1024 .. 12288): the lane-per-block form
+        // costs per pass of R weight rows x 4 activation rows on a compute unit,
+        // the matrix-core form per round of one 32 x 32 tile a compute unit (a
+        // 64 x 64 tile costs two) and super-block. Measured, former and matrix-core
+        // form: Q4_K 4096 x 4096: 12 rows 16.3 / 19.7, 16 rows 22.9 / 19.9, 48 rows
+        // 44.8 / 20.8; 1000 x 12288, 16 rows 26.7 / 44.3; Q6_K 4096 x 4096: 8 rows
+        // 18.2 / 19.4, 12 rows 27.2 / 21.6; 4096 x 12288, 9 rows 68.7 / 50.3.
+        const int64_t cus = device_cus();
+        auto rounds = [&](int64_t t) { return ((M + t - 1) / t * ((N + t - 1) / t) + cus - 1) / cus; };
+        const int64_t small = rounds(32), large = rounds(64), R = kq_rows_per_tile(K);
+        const double passes = double((N + R - 1) / R) * double(M) / (4.0 * double(cus)), over = std::max(0, nb - 32);
+        const double lanes = type == 12 ? 9 + (3 + 0.1 * over) * passes : 10 + (5.2 + 0.06 * over) * passes;
+        const double tiles = (6 + (type == 12 ? 0.83 : 0.92) * nb) * (0.23 + 0.77 * double(std::min(small, 2 * large)));
+        if (tiles <= lanes) {
+            // the small tile takes about half the large one's time for a quarter
+            // of its outputs (Q4_K N 4096, K 4096: 64 rows 21 and 33 us, 509 rows
+            // 98 and 63 us); rows go in slices whose chunk indices fit 32 bits
             auto run = small <= 2 * large ? (type == 12 ? kq_mm<12, 1, 1> : kq_mm<14, 1, 1>) : (type == 12 ? kq_mm<12, 2, 2> : kq_mm<14, 2, 2>);
-            run(wb, ab + r0 * nb * kQ8KBytes, xt + r0 * nb * 64, y + r0 * ldy, resid ? resid + r0 * ldy : nullptr, rows, N, K, ldy, s);
+            const int64_t slice = int64_t(1) << 20;
+            for (int64_t r0 = 0; r0 < M; r0 += slice)
+                run(wb, ab + r0 * nb * kQ8KBytes, xt + r0 * nb * 64, y + r0 * ldy, resid ? resid + r0 * ldy : nullptr, std::min(slice, M - r0), N, K, ldy, s);
+            return;
         }
-        return;
     }
     int R, per;
     kq_plan(M, N, K, kKqTile, &R, &per);
