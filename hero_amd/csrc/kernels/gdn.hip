@@ -643,179 +643,196 @@ __global__ __launch_bounds__(kGdnDim) void gdn_prep_kernel(GdnDecodeArgs a, void
 }
 
 // ---- the token-serial scan, split over value columns and state rows ----------------------
-// The delta rule over the chunk's tokens in order, each value column spread
-// over 16 lanes (one DPP row): the columns of the delta rule are independent
-// (nm/src/recurrent.hpp:146-177), so a workgroup of 256 lanes owns 16 columns
-// and a head takes 8 workgroups. Lane 2s + c of a row holds rows 16s .. 16s+15
-// of its column (segment s); lanes c = 0 run token t+1's decay-and-prediction
-// chain and lanes c = 1 token t's output chain, both over the same updated
-// rows, so one instruction stream advances both chains. A chain visits the
-// segments in row order: segment s adds its 16 terms to the running sum that
-// segment s-1 handed on (a DPP shift by two lanes), so every sum is the
-// reference's left-to-right chain. Both lanes of a segment keep the same
-// copy of the segment's rows. Per token and wave that is 16 rows of updates
-// and products plus the chains' 128 steps, against 128 rows of each for a
-// lane owning a whole column.
-constexpr int kScCols = 16;                  // value columns per workgroup
-constexpr int kScSeg = 8;                    // row segments per column
-constexpr int kScRows = kGdnDim / kScSeg;    // rows per lane (16)
-constexpr int kScTile = 16;                  // tokens per shared-memory tile
-struct ScanColsTile {
-    float k[kScTile][kGdnDim];
-    float q[kScTile][kGdnDim];
-    float v[kScTile][kScCols];
-    float bd[kScTile][2];
+// The delta rule over the chunk's tokens in order. The value columns are
+// independent (nm/src/recurrent.hpp:146-177); a workgroup owns 16 of them (a
+// head takes 8 workgroups) and gives each wave four columns, 16 lanes (one DPP
+// row) per column. Its two chains per token and column are left-to-right sums
+// of 128 rounded products:
+//   pred_t+1 = sum_i (decay S_t)[i] k_t+1[i]   decides delta_t+1: the critical
+//              path, one token after another;
+//   o_t      = sum_i S_t[i] q_t[i]             needed by nobody in the scan.
+// Waves 0-3 run only the predictions. Lane r of a column holds rows 8 r ..
+// 8 r + 7 and their products; the running sum takes sixteen steps, in each of
+// which every lane adds its eight products to what the lane below it had (a
+// DPP shift folded into the first add). Lane r's step r is the chain; its
+// other steps add to sums nobody reads, which costs nothing and saves masking
+// lanes. Per token that is 128 adds, 32 vector instructions of update and
+// product and the delta: ~180 in one instruction stream.
+// Waves 4-7 form the outputs a tile later, from the deltas the first waves left
+// in shared memory, with the same lanes and rows but lane r at token (step - r):
+// there all sixteen lanes' sums count, each its own token's. These waves also
+// stage the inputs.
+//
+// Bound: the prediction chain, 128 dependent adds and 15 shifts with their wait
+// states (~700 clocks of a token). Measured: 1024 tokens, 32 heads 785 -> 395 us
+// (before: both chains in one stream over lane pairs of 16 rows, masked).
+constexpr int kScCols = 16;   // value columns per workgroup
+constexpr int kScTile = 8;    // tokens per barrier
+constexpr int kScRing = 64;   // tokens of inputs held (a power of two)
+constexpr int kScLd = kGdnDim + 4;
+struct ScanShared {
+    float k[kScRing][kScLd];     // padded: lane s reads token t - s, elements 8 s ..
+    float q[kScRing][kScLd];
+    float v[kScRing][kScCols];
+    float delta[kScRing][kScCols];
+    float bd[kScRing][2];
 };
 
-// the running sum of lane i-2 of each row of 16 lanes, in lane i
-__device__ __forceinline__ float row_shr2(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x112, 0xF, 0xF, false));
+// the sum of lane i-1 of each DPP row of 16 lanes, in lane i (lane 0: 0)
+__device__ __forceinline__ float row_shr1(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x111, 0xF, 0xF, true));
 }
-// segment s (lanes 2s, 2s+1 of each row) adds its terms, in row order, to the
-// sum handed on by segment s-1; the final sums end in lanes 14 and 15
-__device__ __forceinline__ float seg_chain(const float (&prod)[kScRows], int seg) {
+// ((0 + prod of row 0) + ...) over the 16 lanes' eight products, in every lane
+__device__ __forceinline__ float row_chain(const float (&prod)[8]) {
     float acc = 0.f;
 #pragma unroll
-    for (int s = 0; s < kScSeg; ++s) {
-        if (seg == s) {
+    for (int s = 0; s < 16; ++s) {
+        if (s > 0) acc = row_shr1(acc);
 #pragma unroll
-            for (int m = 0; m < kScRows; ++m) acc = acc + prod[m];
-        }
-        if (s + 1 < kScSeg) acc = row_shr2(acc);
+        for (int i = 0; i < 8; ++i) acc = acc + prod[i];
     }
-    return acc;
-}
-// lane 14 of each row of the wave, in every lane of that row
-__device__ __forceinline__ float row_lane14(float v, int row) {
-    const int b = __float_as_int(v);
-    const int r0 = __builtin_amdgcn_readlane(b, 14), r1 = __builtin_amdgcn_readlane(b, 30);
-    const int r2 = __builtin_amdgcn_readlane(b, 46), r3 = __builtin_amdgcn_readlane(b, 62);
-    return __int_as_float(row == 0 ? r0 : row == 1 ? r1 : row == 2 ? r2 : r3);
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(acc), 0x15F, 0xF, 0xF, true));  // lane 15's
 }
 
-__global__ __launch_bounds__(256) void gdn_scan_cols_kernel(GdnDecodeArgs a, void* ws) {
-    const int lane = threadIdx.x;
+__global__ __launch_bounds__(512) void gdn_scan_cols_kernel(GdnDecodeArgs a, void* ws) {
+    extern __shared__ __align__(16) uint8_t scan_smem[];
+    ScanShared& sh = *reinterpret_cast<ScanShared*>(scan_smem);
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int h = blockIdx.x / (kGdnDim / kScCols), c0 = (blockIdx.x % (kGdnDim / kScCols)) * kScCols, hk = h % a.Hk;
-    const int jl = lane / 16, seg = (lane % 16) / 2, ch = lane % 2, row = (lane % 64) / 16;
-    const int j = c0 + jl, r0 = seg * kScRows;
     const int T = a.B;
     if (a.positions[0] < 0) return;
     const GdnPrefillWork w = gdn_work(ws, T, a.Hk, a.Hv);
-    float* S = a.state + int64_t(h) * kGdnState + j;
-    __shared__ __align__(16) ScanColsTile tiles[2];
-    const int ntiles = (T + kScTile - 1) / kScTile;
+    const int r = lane & 15, cl = 4 * (wave & 3) + (lane >> 4);  // lane of the column, column of the workgroup
+    float* S = a.state + int64_t(h) * kGdnState + c0 + cl;
+    constexpr int kMask = kScRing - 1;
 
-    // a tile: k and q (2 float4 each per lane), v of the 16 columns (lanes
-    // 0..63) and (beta, decay) (lanes 64..79); zeros past the last token
-    float4 pk[2], pq[2], pv = make_float4(0.f, 0.f, 0.f, 0.f);
-    float2 pbd = make_float2(0.f, 0.f);
+    // staging by waves 4-7: thread st loads one float4 of k and of q per tile
+    const int st = tid - 256;
+    float4 pk, pq, pv;
+    float2 pbd;
     auto load = [&](int tile) {
-        const int t0 = tile * kScTile;
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int f = lane + 256 * u, tt = t0 + f / (kGdnDim / 4), c4 = f % (kGdnDim / 4);
-            const int64_t o = (int64_t(tt) * a.Hk + hk) * kGdnDim;
-            pk[u] = tt < T ? reinterpret_cast<const float4*>(w.k + o)[c4] : make_float4(0.f, 0.f, 0.f, 0.f);
-            pq[u] = tt < T ? reinterpret_cast<const float4*>(w.q + o)[c4] : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-        if (lane < 64) {
-            const int tt = t0 + lane / 4;
-            pv = tt < T ? reinterpret_cast<const float4*>(w.v + (int64_t(tt) * a.Hv + h) * kGdnDim + c0)[lane % 4] : make_float4(0.f, 0.f, 0.f, 0.f);
-        } else if (lane < 64 + kScTile) {
-            const int tt = t0 + lane - 64;
-            pbd = tt < T ? reinterpret_cast<const float2*>(w.bd)[int64_t(tt) * a.Hv + h] : make_float2(0.f, 0.f);
+        const int t = tile * kScTile + st / (kGdnDim / 4), c4 = st % (kGdnDim / 4);
+        const int64_t o = (int64_t(min(t, T - 1)) * a.Hk + hk) * kGdnDim;
+        pk = reinterpret_cast<const float4*>(w.k + o)[c4];
+        pq = reinterpret_cast<const float4*>(w.q + o)[c4];
+        if (st < kScTile * kScCols / 4) {
+            const int tv = min(tile * kScTile + st / (kScCols / 4), T - 1);
+            pv = reinterpret_cast<const float4*>(w.v + (int64_t(tv) * a.Hv + h) * kGdnDim + c0)[st % (kScCols / 4)];
+        } else if (st >= 64 && st < 64 + kScTile) {
+            pbd = reinterpret_cast<const float2*>(w.bd)[int64_t(min(tile * kScTile + st - 64, T - 1)) * a.Hv + h];
         }
     };
-    auto store = [&](ScanColsTile& dst) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            reinterpret_cast<float4*>(&dst.k[0][0])[lane + 256 * u] = pk[u];
-            reinterpret_cast<float4*>(&dst.q[0][0])[lane + 256 * u] = pq[u];
-        }
-        if (lane < 64)
-            reinterpret_cast<float4*>(&dst.v[0][0])[lane] = pv;
-        else if (lane < 64 + kScTile)
-            reinterpret_cast<float2*>(&dst.bd[0][0])[lane - 64] = pbd;
-    };
-    auto rows16 = [&](const float* src, float (&dst)[kScRows]) {
-        const float4* s4 = reinterpret_cast<const float4*>(src + r0);
-#pragma unroll
-        for (int u = 0; u < kScRows / 4; ++u) {
-            const float4 x = s4[u];
-            dst[4 * u] = x.x, dst[4 * u + 1] = x.y, dst[4 * u + 2] = x.z, dst[4 * u + 3] = x.w;
-        }
+    auto store = [&](int tile) {
+        const int t = (tile * kScTile + st / (kGdnDim / 4)) & kMask, c4 = st % (kGdnDim / 4);
+        *reinterpret_cast<float4*>(&sh.k[t][4 * c4]) = pk;
+        *reinterpret_cast<float4*>(&sh.q[t][4 * c4]) = pq;
+        if (st < kScTile * kScCols / 4)
+            *reinterpret_cast<float4*>(&sh.v[(tile * kScTile + st / (kScCols / 4)) & kMask][4 * (st % (kScCols / 4))]) = pv;
+        else if (st >= 64 && st < 64 + kScTile)
+            *reinterpret_cast<float2*>(sh.bd[(tile * kScTile + st - 64) & kMask]) = pbd;
     };
 
-    float col[kScRows];  // S[r0 + m][j]
-#pragma unroll
-    for (int m = 0; m < kScRows; ++m) col[m] = S[int64_t(r0 + m) * kGdnDim];
-    load(0);
-    store(tiles[0]);
-    if (ntiles > 1) {
+    const int phases = (T + 15 + kScTile - 1) / kScTile + 1;  // the outputs end 15 steps and a tile after the predictions
+    if (wave >= 4) {
+        load(0);
+        store(0);
         load(1);
-        store(tiles[1]);
+        store(1);
+        load(2);
     }
-    if (ntiles > 2) load(2);
     __syncthreads();
 
-    // token 0: decay and prediction chain (nm/src/recurrent.hpp:152-160)
-    float delta;
-    {
-        float kk[kScRows], prod[kScRows];
-        rows16(tiles[0].k[0], kk);
-        const float dec = tiles[0].bd[0][1];
+    if (wave < 4) {
+        __builtin_amdgcn_s_setprio(3);
+        float col[8], kc[8];  // S[8 r + m][column], k[8 r + m]
+        auto keys = [&](int t, float (&k)[8]) {
+            const float4* p = reinterpret_cast<const float4*>(sh.k[t & kMask] + 8 * r);
+            const float4 x = p[0], y = p[1];
+            k[0] = x.x, k[1] = x.y, k[2] = x.z, k[3] = x.w, k[4] = y.x, k[5] = y.y, k[6] = y.z, k[7] = y.w;
+        };
 #pragma unroll
-        for (int m = 0; m < kScRows; ++m) {
-            col[m] = col[m] * dec;
-            prod[m] = col[m] * kk[m];
-        }
-        const float pred = row_lane14(seg_chain(prod, seg), row);
-        delta = (tiles[0].v[0][jl] - pred) * tiles[0].bd[0][0];
-    }
-    for (int t = 0; t < T; ++t) {
-        const int tile = t / kScTile, r = t % kScTile;
-        if (r == 0 && tile > 0) {
-            // tile-1's buffer is free: it takes tile+1 (loaded a tile ago)
-            __syncthreads();
-            if (tile + 1 < ntiles) store(tiles[(tile + 1) & 1]);
-            if (tile + 2 < ntiles) load(tile + 2);
-            __syncthreads();
-        }
-        const ScanColsTile& cur = tiles[tile & 1];
-        const ScanColsTile& nxt = tiles[((t + 1) / kScTile) & 1];
-        const int rn = (t + 1) % kScTile;
-        float kc[kScRows], f[kScRows], prod[kScRows];
-        rows16(cur.k[r], kc);
-        // lanes c = 0: token t+1's key (zeros past the last token); c = 1: token t's query
-        rows16(ch == 0 ? nxt.k[rn] : cur.q[r], f);
-        float o;
-        if (t + 1 < T) {
-            const float dec = nxt.bd[rn][1];
+        for (int m = 0; m < 8; ++m) col[m] = S[int64_t(8 * r + m) * kGdnDim];
+        // token 0: decay and prediction chain (nm/src/recurrent.hpp:152-160)
+        keys(0, kc);
+        float pred;
+        {
+            const float dec = sh.bd[0][1];
+            float prod[8];
 #pragma unroll
-            for (int m = 0; m < kScRows; ++m) {
-                const float v = col[m] + kc[m] * delta;  // S[i][j] += k[i] * delta
-                const float vd = v * dec;                // next token: S[i][j] *= decay
-                col[m] = vd;
-                prod[m] = (ch == 0 ? vd : v) * f[m];     // pred += S[i][j] * k'[i]  |  o += S[i][j] * q[i]
+            for (int m = 0; m < 8; ++m) {
+                col[m] = col[m] * dec;
+                prod[m] = col[m] * kc[m];
             }
-            const float acc = seg_chain(prod, seg);
-            o = acc;
-            const float pred = row_lane14(acc, row);
-            delta = (nxt.v[rn][jl] - pred) * nxt.bd[rn][0];
-        } else {
-#pragma unroll
-            for (int m = 0; m < kScRows; ++m) {
-                const float v = col[m] + kc[m] * delta;
-                col[m] = v;
-                prod[m] = v * f[m];
-            }
-            o = seg_chain(prod, seg);
+            pred = row_chain(prod);
         }
-        if (lane % 16 == 15) w.o[(int64_t(t) * a.Hv + h) * kGdnDim + j] = o;
-    }
-    if (ch == 1) {
+        float delta = (sh.v[0][cl] - pred) * sh.bd[0][0];
+        sh.delta[0][cl] = delta;
+        // the inputs of token t + 1 are read a token ahead
+        float kn[8];
+        keys(1, kn);
+        float vn = sh.v[1][cl], bn = sh.bd[1][0], dn = sh.bd[1][1];
+        auto token = [&](int t) {  // token t's update, token t + 1's prediction
+            float kf[8], prod[8];
+            keys(t + 2, kf);
+            const float vf = sh.v[(t + 2) & kMask][cl], bf = sh.bd[(t + 2) & kMask][0], df = sh.bd[(t + 2) & kMask][1];
 #pragma unroll
-        for (int m = 0; m < kScRows; ++m) S[int64_t(r0 + m) * kGdnDim] = col[m];
+            for (int m = 0; m < 8; ++m) {
+                const float x = (col[m] + kc[m] * delta) * dn;  // S[i][j] += k[i] * delta, then token t + 1's decay
+                col[m] = x;
+                prod[m] = x * kn[m];
+            }
+            pred = row_chain(prod);
+            delta = (vn - pred) * bn;
+            sh.delta[(t + 1) & kMask][cl] = delta;  // the same value from the column's 16 lanes
+#pragma unroll
+            for (int m = 0; m < 8; ++m) kc[m] = kn[m], kn[m] = kf[m];
+            vn = vf, bn = bf, dn = df;
+        };
+        for (int j = 0; j < phases; ++j) {
+            const int t0 = kScTile * j;
+            if (t0 + kScTile < T) {
+#pragma unroll
+                for (int u = 0; u < kScTile; ++u) token(t0 + u);
+            } else if (t0 < T) {
+                for (int t = t0; t + 1 < T; ++t) token(t);
+#pragma unroll
+                for (int m = 0; m < 8; ++m) S[int64_t(8 * r + m) * kGdnDim] = col[m] + kc[m] * delta;
+            }
+            __syncthreads();
+        }
+    } else {
+        float col[8];  // S[8 r + i][column] at this lane's token
+#pragma unroll
+        for (int i = 0; i < 8; ++i) col[i] = S[int64_t(8 * r + i) * kGdnDim];
+        float acc = 0.f;
+        for (int j = 0; j < phases; ++j) {
+            store(j + 2);
+            load(j + 3);
+            if (j > 0) {
+#pragma unroll 2
+                for (int u = 0; u < kScTile; ++u) {
+                    const int t = kScTile * (j - 1) + u - r, slot = t & kMask;
+                    // lane r - 1's sum of the same token; the first lane starts at 0
+                    acc = row_shr1(acc);
+                    if (t >= 0 && t < T) {
+                        const float4* kp = reinterpret_cast<const float4*>(&sh.k[slot][8 * r]);
+                        const float4* qp = reinterpret_cast<const float4*>(&sh.q[slot][8 * r]);
+                        const float4 k0 = kp[0], k1 = kp[1], q0 = qp[0], q1 = qp[1];
+                        const float kk[8] = {k0.x, k0.y, k0.z, k0.w, k1.x, k1.y, k1.z, k1.w};
+                        const float qq[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+                        const float dec = sh.bd[slot][1], delta = sh.delta[slot][cl];
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) {
+                            const float x = col[i] * dec + kk[i] * delta;
+                            col[i] = x;
+                            acc = acc + x * qq[i];
+                        }
+                        if (r == 15) w.o[(int64_t(t) * a.Hv + h) * kGdnDim + c0 + cl] = acc;
+                    }
+                }
+            }
+            __syncthreads();
+        }
     }
 }
 
@@ -1204,7 +1221,7 @@ void launch_gdn_prefill(const GdnDecodeArgs& a, void* work, hipStream_t s, bool 
         hipLaunchKernelGGL(gdn_chunk_scan_kernel, dim3(unsigned(a.Hv), unsigned(kGdnDim / kChunkCols)), dim3(256), kChunkScanShared, s, a, work);
     }
     else
-        hipLaunchKernelGGL(gdn_scan_cols_kernel, dim3(unsigned(a.Hv * (kGdnDim / kScCols))), dim3(256), 0, s, a, work);
+        hipLaunchKernelGGL(gdn_scan_cols_kernel, dim3(unsigned(a.Hv * (kGdnDim / kScCols))), dim3(512), sizeof(ScanShared), s, a, work);
     hipLaunchKernelGGL(gdn_out_kernel, dim3(unsigned(a.Hv), unsigned(a.B)), dim3(kGdnDim), 0, s, a, work);
     const int64_t CC = 2 * int64_t(a.Hk) * kGdnDim + int64_t(a.Hv) * kGdnDim;
     const int64_t n = int64_t(std::min(a.B, a.W)) * CC;

@@ -490,6 +490,13 @@ def test_gdn_prefill_chunks_match_oracle(lib, W, chunks):
         pos += T
 
 
+# chunk lengths around the scan's 8-token tiles, its 16-lane output skew and the
+# 64-token ring of inputs it wraps (bit for bit, as the test above)
+@pytest.mark.parametrize("chunks", [[8, 9, 15, 16], [17, 24, 23], [64, 65], [143]])
+def test_gdn_prefill_scan_tile_edges_match_oracle(lib, chunks):
+    test_gdn_prefill_chunks_match_oracle(lib, 4, chunks)
+
+
 @pytest.mark.parametrize("T,hk,hv", [(70, 2, 4), (300, 4, 4)])
 def test_gdn_chunked_prefill_matches_serial(lib, T, hk, hv):
     """The chunked (WY) delta-net prefill against the token-serial one (which
