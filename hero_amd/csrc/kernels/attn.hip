@@ -1062,178 +1062,466 @@ __global__ __launch_bounds__(NT) void attn_softmax_regs_kernel(AttnDecodeArgs a)
     }
 }
 
-// out[c] = sum_j alpha_j * v_j[c] (rows in order, core.hpp:206-208) for a
-// block of R consecutive rows of one sequence (a prefill chunk, full causal
-// visibility), all query heads of one K/V group chunk (up to 4) and all 128
-// channels: each V row and each weight is read from memory once per block
-// instead of once per row and head. Wave w owns channels 32 w .. 32 w + 31;
-// lane l owns row r = l % R and channels 32 w + CPL (l / R) .. + CPL - 1 of
-// every head of the chunk (4 x CPL chains in registers). 32-key tiles of V
-// ([key][128 channels]) and of the weights ([key quad][head, row][4 keys])
-// land in shared memory through global_load_lds, two buffers deep; per key a
-// lane reads its CPL channels (all lanes with the same channel group share
-// the address) and, per 4 keys, one 16-byte weight read per head (lanes
-// of consecutive rows read consecutive addresses), then does 8 CPL fp32
-// operations. A row only adds keys at or before its position (the tiles past
-// the block's first position test it per lane). Then the gate and the Q8_0
-// block of 32 channels (spread over 32 / CPL lanes) as attn_pv_kernel.
-// The host runs it for window 0 and max_ctx % 4 == 0 (16-byte aligned
-// weight quads and V rows).
-constexpr int kPrRows = 8;                         // rows per workgroup (16 measured 2% slower over a 2048-token prefill)
+// ---- prefill over the shared cache: blocks of (row, query head) pairs ------------------------
+// Consecutive rows see nearly the same keys and a K/V group's query heads the
+// same ones, so a block of pairs (hp heads, the group's up to 4, of some rows)
+// is worked off together. Scores and weighted sums are chains of rounded
+// products: a multiply and an add per pair, channel and key, nothing to
+// contract. Each lane therefore keeps a tile of chains in registers -- 8 pairs x
+// 4 keys of scores, 4 pairs x 4 channels of the sums -- so that a
+// 16-byte shared-memory read, whose 64 lanes take the unit as long as four
+// vector instructions, feeds 16 or more of those.
+//
+// Bound: vector instructions, 4.5 clocks of a SIMD for 64 multiplies and adds.
+// 1024 rows after 1024 cached, 32 heads of 128, 8 K/V heads: 6.4 G
+// multiply-adds, 187 us at 2.35 GHz (the clock drops to ~2 GHz under them), for
+// each of the two products. Measured, former kernels in brackets: scores 302
+// [403], softmax 127 [325], weighted sum 313 [330]; the whole call 735 [1045].
+// Depth-1 fp32 MFMAs in place of the multiplies were no faster (scores 284,
+// sums 346 us): they hold the vector units, and two waves' adds then seldom run
+// side by side.
+constexpr int kRbPairs = 32;  // pairs of a score block
+
+// query heads of a block (a power of two) and blocks per K/V group
+__host__ __device__ inline int rb_heads(int group) { return group >= 3 ? 4 : group; }
+__host__ __device__ inline int rb_chunks(int group) { return (group + rb_heads(group) - 1) / rb_heads(group); }
+
+// scores of 256-key tiles: wave w forms pairs 8 w .. 8 w + 7, lane l keys 4 l ..
+// 4 l + 3. K is cached channel-major, so a channel of the tile is one 1 KB read
+// the four waves share through L1; eight channels are read ahead. The pairs'
+// queries stay in shared memory, [channel][pair]. Score t of a pair is key
+// first + t, first the pair's first visible key. Workgroup z takes tiles z,
+// z + gridDim.z, ...
+template <int DH>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void attn_scores_rows_kernel(AttnDecodeArgs a) {
+    __shared__ __align__(16) float qs[DH * kRbPairs];
+    __shared__ int4 see[kRbPairs];  // each pair's visible keys x .. y (y < x: none), its row of scores z
+    const int tid = int(threadIdx.x), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int group = a.Hq / a.Hkv, hp = rb_heads(group), chunks = rb_chunks(group), R = kRbPairs / hp;
+    const int g = int(blockIdx.x) / chunks, h0 = g * group + (int(blockIdx.x) % chunks) * hp;
+    const int nh = min(hp, (g + 1) * group - h0);
+    const int row0 = (int(gridDim.y) - 1 - int(blockIdx.y)) * R;  // the longest rows first
+    int key_lo = INT32_MAX, key_hi = -1;
+    for (int r = 0; r < R && row0 + r < a.B; ++r) {
+        const int p = a.positions[row0 + r];
+        if (p < 0 || p >= a.max_ctx) continue;
+        key_lo = min(key_lo, visible_first(p, a.window));
+        key_hi = max(key_hi, p);
+    }
+    if (key_hi < 0) return;
+    key_lo &= ~3;  // aligned 16-byte reads (where max_ctx allows)
+    const int ntiles = (key_hi - key_lo) / 256 + 1;
+    if (int(blockIdx.z) >= ntiles) return;
+    if (tid < kRbPairs) {
+        const int r = row0 + tid / hp;
+        const int p = r < a.B && tid % hp < nh ? a.positions[r] : -1;
+        const bool ok = p >= 0 && p < a.max_ctx;
+        see[tid] = make_int4(ok ? visible_first(p, a.window) : 0, ok ? p : -1, r * a.Hq + h0 + tid % hp, 0);
+    }
+    for (int i = tid; i < kRbPairs * (DH / 4); i += 256) {
+        const int pair = i % kRbPairs, c4 = i / kRbPairs;
+        const int r = min(row0 + pair / hp, a.B - 1), h = h0 + min(pair % hp, nh - 1);
+        const float4 q = reinterpret_cast<const float4*>(a.q_rot + (int64_t(r) * a.Hq + h) * DH)[c4];
+        float* d = qs + 4 * c4 * kRbPairs + pair;
+        d[0] = q.x, d[kRbPairs] = q.y, d[2 * kRbPairs] = q.z, d[3 * kRbPairs] = q.w;
+    }
+    __syncthreads();
+    const float* kh = a.k_cache + int64_t(g) * DH * a.max_ctx;
+    const float4* qw = reinterpret_cast<const float4*>(qs + 8 * wave);
+
+    auto tile_scores = [&](int key0, auto whole) {
+        const int kl = key0 + 4 * lane;
+        auto key4 = [&](int c) {
+            const float* k = kh + int64_t(c) * a.max_ctx;
+            float4 v;
+            if constexpr (decltype(whole)::value) {
+                __builtin_memcpy(&v, reinterpret_cast<const uint8_t*>(k) + uint32_t(4 * kl), 16);  // a uniform base and a 32-bit offset
+            } else {  // the tile runs past the cache
+                const int last = int(a.max_ctx) - 1;
+                v = make_float4(k[min(kl, last)], k[min(kl + 1, last)], k[min(kl + 2, last)], k[min(kl + 3, last)]);
+            }
+            return v;
+        };
+        float acc[8][4];
+#pragma unroll
+        for (int p = 0; p < 8; ++p)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[p][e] = 0.f;
+        float4 kn[8], q0 = qw[0], q1 = qw[1];  // the next eight channels of the keys, the next channel of the queries
+#pragma unroll
+        for (int u = 0; u < 8; ++u) kn[u] = key4(u);
+#pragma unroll 1
+        for (int c = 0; c < DH; c += 8) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const float k[4] = {kn[u].x, kn[u].y, kn[u].z, kn[u].w};
+                const float q[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+                kn[u] = key4(min(c + 8 + u, DH - 1));
+                const float4* qx = qw + min(c + u + 1, DH - 1) * (kRbPairs / 4);
+                q0 = qx[0], q1 = qx[1];
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int p = 0; p < 8; ++p)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[p][e] += q[p] * k[e];
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < 8; ++p) {
+            const int4 s = see[8 * wave + p];
+            float* d = a.scores + int64_t(s.z) * a.max_ctx + kl - s.x;
+            const float4 v = make_float4(a.score_scale * acc[p][0], a.score_scale * acc[p][1], a.score_scale * acc[p][2], a.score_scale * acc[p][3]);
+            if (kl >= s.x && kl + 3 <= s.y) {
+                __builtin_memcpy(d, &v, 16);
+            } else {
+                if (kl >= s.x && kl <= s.y) d[0] = v.x;
+                if (kl + 1 >= s.x && kl + 1 <= s.y) d[1] = v.y;
+                if (kl + 2 >= s.x && kl + 2 <= s.y) d[2] = v.z;
+                if (kl + 3 >= s.x && kl + 3 <= s.y) d[3] = v.w;
+            }
+        }
+    };
+    for (int tile = int(blockIdx.z); tile < ntiles; tile += int(gridDim.z)) {
+        const int key0 = key_lo + 256 * tile;
+        if (key0 + 256 <= a.max_ctx)
+            tile_scores(key0, std::true_type{});
+        else
+            tile_scores(key0, std::false_type{});
+    }
+}
+
+// The softmax numerators and totals of eight (row, head) pairs: the max over each
+// pair's scores, e_j = exp(s_j - max) written back in place, and their sum in
+// index order as a plain chain, one lane per pair: with the pairs side by side
+// the chain costs less than finding the same sum in parallel
+// (hero/seqsum.hpp). The waves form tile k + 1's exponentials while one of them
+// (they take turns) adds tile k's from shared memory. Totals go to q_rot (the
+// scores are formed, its contents are no longer needed); the weighted sum
+// divides as it reads. Any number of keys.
+constexpr int kSrLd = 64 + 4;
+constexpr int kSrPairs = 8;  // two per wave (eight per wave: 2-8% slower calls, up to a fifth for few rows)
+__global__ __launch_bounds__(256) void attn_softmax_rows_kernel(AttnDecodeArgs a) {
+    constexpr int PW = kSrPairs / 4, NP = kSrPairs;
+    __shared__ __align__(16) float eb[2][NP][kSrLd];
+    __shared__ uint64_t etab[32];
+    __shared__ float total[NP];
+    __shared__ int count[NP];
+    const int tid = int(threadIdx.x), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t pairs = int64_t(a.B) * a.Hq, pair0 = (int64_t(gridDim.x) - 1 - blockIdx.x) * NP;  // the longest rows first
+    if (tid < NP) {
+        int n = 0;
+        if (pair0 + tid < pairs) {
+            const int p = a.positions[(pair0 + tid) / a.Hq];
+            if (p >= 0 && p < a.max_ctx) n = p + 1 - visible_first(p, a.window);
+        }
+        count[tid] = n;
+        total[tid] = 0.f;
+    }
+    fill_exp_table(etab, tid);
+    __syncthreads();
+    const ExpTab ex{etab};
+    int n[PW], nmax = 0;
+#pragma unroll
+    for (int i = 0; i < PW; ++i) n[i] = __builtin_amdgcn_readfirstlane(count[PW * wave + i]);
+#pragma unroll
+    for (int i = 0; i < NP; ++i) nmax = max(nmax, count[i]);
+    nmax = __builtin_amdgcn_readfirstlane(nmax);
+    float* sc = a.scores + (pair0 + PW * wave) * a.max_ctx;  // this wave's pairs
+    float s[PW], mx[PW];
+    auto load = [&](int t) {
+#pragma unroll
+        for (int i = 0; i < PW; ++i) s[i] = t < n[i] ? sc[int64_t(i) * a.max_ctx + t] : -INFINITY;
+    };
+#pragma unroll
+    for (int i = 0; i < PW; ++i) mx[i] = -INFINITY;
+    for (int t = lane; t < nmax; t += 64) {
+        load(t);
+#pragma unroll
+        for (int i = 0; i < PW; ++i) mx[i] = fmaxf(mx[i], s[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < PW; ++i)
+        for (int off = 32; off > 0; off >>= 1) mx[i] = fmaxf(mx[i], __shfl_xor(mx[i], off));
+    const int tiles = (nmax + 63) / 64;
+    if (tiles > 0) load(lane);
+    for (int k = 0; k <= tiles; ++k) {
+        if (k < tiles) {
+            const int t = 64 * k + lane;
+            float e[PW];
+#pragma unroll
+            for (int i = 0; i < PW; ++i) e[i] = s[i];
+            load(t + 64);
+#pragma unroll
+            for (int i = 0; i < PW; ++i) {
+                e[i] = t < n[i] ? ex.exp(e[i] - mx[i]) : 0.f;
+                eb[k & 1][PW * wave + i][lane] = e[i];
+                if (t < n[i]) sc[int64_t(i) * a.max_ctx + t] = e[i];
+            }
+        }
+        __syncthreads();
+        if (k < tiles && wave == (k & 3) && lane < NP) {
+            float acc = total[lane];
+            const float4* row = reinterpret_cast<const float4*>(eb[k & 1][lane]);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const float4 v = row[j];
+                acc += v.x;
+                acc += v.y;
+                acc += v.z;
+                acc += v.w;
+            }
+            total[lane] = acc;
+        }
+    }
+    if (tid < NP && pair0 + tid < pairs) a.q_rot[pair0 + tid] = total[tid];
+}
+
+// out[c] = sum_j alpha_j * v_j[c] (rows in order, core.hpp:206-208),
+// alpha_j = e_j / total, for a block of 16 PL pairs and 128 channels. Half-wave s
+// (of sixteen) owns pairs PL s .. PL s + PL - 1, its lane l channels 4 l .. 4 l + 3.
+// Four pairs a lane: eight halve the shared-memory reads, but their workgroups
+// leave two waves a SIMD, of which the longer ends alone (400 against 313 us).
+// Workgroups of eight waves: with four, the waves of the workgroups a compute
+// unit holds paired unevenly on its SIMDs (346 us).
+// Tiles of 32 keys, two buffers: V through global_load_lds as [key][channel],
+// the weights read, divided (once per pair and key and channel part) and stored
+// as [key][pair ^ 4 (key / 4)] (the eight lanes of a pair store to banks of their
+// own). Tiles some pair sees only in part test each key. Then the gate
+// and the Q8_0 blocks of 32 channels.
 constexpr int kPrKeys = 32;                        // keys per tile
-constexpr int kPrThreads = 256;                    // four waves: 32 channels each
-constexpr int kPrHeads = 4;                        // query heads per workgroup
+constexpr int kPrThreads = 512;
 constexpr int kPrVQuads = kPrKeys * kAttnDim / 4;  // 16-byte pieces of a V tile: 1024
 
-template <int R, int DH>
-__global__ __launch_bounds__(kPrThreads) void attn_pv_rows_kernel(AttnDecodeArgs a) {
+template <int DH, int PL>
+__global__ __launch_bounds__(kPrThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void attn_pv_rows_kernel(AttnDecodeArgs a) {
     constexpr int kParts = DH / kAttnDim;  // 128-channel parts of a head (one workgroup each)
-    constexpr int CG = 64 / R;          // channel groups per wave
-    constexpr int CPL = 32 / CG;        // channels per lane
-    constexpr int NP = kPrHeads * R;    // (head, row) pairs
-    constexpr int AQuads = kPrKeys / 4 * NP;  // 16-byte pieces of a weight tile
-    static_assert(CPL % 4 == 0 && AQuads % kPrThreads == 0 && kPrVQuads % kPrThreads == 0, "tile geometry");
-    __shared__ __align__(16) float vt[2][kPrKeys * kAttnDim];  // [key][channel]
-    __shared__ __align__(16) float at[2][AQuads * 4];          // [key quad][head * R + row][4 keys]
-
-    const int tid = int(threadIdx.x), wave = tid / 64, lane = tid % 64;
-    const int r = lane % R, cg = lane / R;
-    const int group = a.Hq / a.Hkv, nchunk = (group + kPrHeads - 1) / kPrHeads;
-    const int part = int(blockIdx.x) % kParts, gcx = int(blockIdx.x) / kParts;
-    const int g = gcx / nchunk, h0 = g * group + (gcx % nchunk) * kPrHeads;
-    const int nh = min(kPrHeads, g * group + group - h0);
-    const int row0 = int(blockIdx.y) * R;
-    const int nrows = min(R, a.B - row0);
-    // the block's positions: the first row's (every row sees keys up to it)
-    // and the largest (the last tile)
-    const int my_row = row0 + min(r, nrows - 1);
-    const int my_pos = r < nrows ? a.positions[my_row] : -1;
-    int pos_lo = INT32_MAX, pos_hi = -1;
-    for (int i = 0; i < nrows; ++i) {
-        const int p = a.positions[row0 + i];
-        pos_lo = min(pos_lo, p);
-        pos_hi = max(pos_hi, p);
+    constexpr int NP = kPrThreads / 32 * PL;
+    static_assert(kPrKeys % 4 == 0 && kPrKeys <= 32 && 8 * NP <= kPrThreads, "one weight quad per thread");
+    __shared__ __align__(16) float vt[2][kPrKeys * kAttnDim];
+    __shared__ __align__(16) float at[2][kPrKeys * NP];
+    const int tid = int(threadIdx.x), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int group = a.Hq / a.Hkv, hp = rb_heads(group), chunks = rb_chunks(group), R = NP / hp;
+    const int part = int(blockIdx.x) % kParts, gc = int(blockIdx.x) / kParts;
+    const int g = gc / chunks, h0 = g * group + (gc % chunks) * hp;
+    const int nh = min(hp, (g + 1) * group - h0);
+    // later rows see more keys: two neighbouring row blocks of the grid, and two
+    // half of it apart, take one from either end, so that those a compute unit
+    // gets add up to much the same either way
+    const int y = int(blockIdx.y), half = int(gridDim.y) / 2, k2 = y < half ? y : y - half;
+    const int row0 = (y >= 2 * half ? y : (k2 % 2 == 0) == (y < half) ? k2 : 2 * half - 1 - k2) * R;
+    // visible keys of a pair: lo .. hi (hi < lo: none)
+    auto visible = [&](int pair, int& lo, int& hi) {
+        const int r = row0 + pair / hp;
+        const int p = r < a.B && pair % hp < nh ? a.positions[r] : -1;
+        const bool ok = p >= 0 && p < a.max_ctx;
+        lo = ok ? visible_first(p, a.window) : 0;
+        hi = ok ? p : -1;
+    };
+    int key_lo = INT32_MAX, key_hi = -1, all_lo = 0, all_hi = INT32_MAX;  // keys some row sees, keys every row sees
+    for (int r = 0; r < R; ++r) {
+        int lo, hi;
+        visible(r * hp, lo, hi);
+        all_lo = max(all_lo, lo), all_hi = min(all_hi, hi);
+        if (hi >= 0) key_lo = min(key_lo, lo), key_hi = max(key_hi, hi);
     }
-    if (pos_hi < 0 || pos_hi >= a.max_ctx || pos_lo < 0) return;  // the host keeps positions in range
-    const int ntiles = (pos_hi + kPrKeys) / kPrKeys;
-    const int full_tiles = (pos_lo + 1) / kPrKeys;  // tiles every row of the block sees whole
+    if (key_hi < 0) return;
+    if (nh < hp) all_hi = -1;
+    const int tile0 = key_lo / kPrKeys, tile1 = key_hi / kPrKeys;
     const int64_t kw = int64_t(a.Hkv) * DH;
     const float* vb = a.v_cache + int64_t(g) * DH + part * kAttnDim;  // shared cache: sequence 0; this part's channels
 
-    // staging: V piece q = key q / 32, channels 4 (q % 32) ..; weight piece
-    // q = key quad q / NP, pair q % NP = head * R + row; rows past the block and
-    // heads past nh read the last valid ones, keys past the cache its last
-    // rows (never used)
+    // staging: this thread's weights are pair tid / 8, keys 4 (tid % 8) ..
+    const int squad = tid % 8, spair = min(tid / 8, NP - 1);
+    const bool stager = tid < 8 * NP && squad < kPrKeys / 4;
+    int slo, shi;
+    visible(spair, slo, shi);
+    if (!stager) shi = -1;
+    const int64_t sidx = int64_t(min(row0 + spair / hp, a.B - 1)) * a.Hq + h0 + min(spair % hp, nh - 1);
+    const float* srow = a.scores + sidx * a.max_ctx;
+    const float stotal = a.q_rot[sidx], srcp = 1.f / stotal;
+    const float* vsrc[kPrVQuads / kPrThreads];  // this thread's pieces of the next tile
+#pragma unroll
+    for (int k = 0; k < kPrVQuads / kPrThreads; ++k) vsrc[k] = vb + int64_t(tile0 * kPrKeys + k * (kPrThreads / 32) + tid / 32) * kw + 4 * (tid % 32);
+    float ev[4];
     auto issue = [&](int tile) {
         const int j0 = tile * kPrKeys;
         float* vdst = vt[tile & 1];
-        float* adst = at[tile & 1];
+        const bool inside = j0 + kPrKeys <= int(a.max_ctx);
 #pragma unroll
         for (int k = 0; k < kPrVQuads / kPrThreads; ++k) {
-            const int q = k * kPrThreads + tid;
-            const int key = min(j0 + q / 32, int(a.max_ctx) - 1);
-            lds_dma_b128(vb + int64_t(key) * kw + 4 * (q % 32), lds_offset(vdst + 4 * (k * kPrThreads + wave * 64)));
+            const int key = j0 + k * (kPrThreads / 32) + tid / 32;
+            // keys past the cache read its last row (never used)
+            const float* src = inside || key < int(a.max_ctx) ? vsrc[k] : vb + (a.max_ctx - 1) * kw + 4 * (tid % 32);
+            lds_dma_b128(src, lds_offset(vdst + 4 * (k * kPrThreads + wave * 64)));
+            vsrc[k] += kPrKeys * kw;
         }
+        const int key = j0 + 4 * squad;
+        if (stager && j0 >= all_lo && j0 + kPrKeys - 1 <= all_hi) {
+            __builtin_memcpy(ev, srow + (key - slo), 16);  // 4-byte aligned
+        } else {
 #pragma unroll
-        for (int k = 0; k < AQuads / kPrThreads; ++k) {
-            const int q = k * kPrThreads + tid;
-            const int pair = q % NP, kq = q / NP;
-            const int hh = min(pair / R, nh - 1), rr = min(pair % R, nrows - 1);
-            const int key = min(j0 + 4 * kq, int(a.max_ctx) - 4);
-            const float* src = a.scores + (int64_t(row0 + rr) * a.Hq + h0 + hh) * a.max_ctx + key;
-            lds_dma_b128(src, lds_offset(adst + 4 * (k * kPrThreads + wave * 64)));
+            for (int u = 0; u < 4; ++u) ev[u] = key + u >= slo && key + u <= shi ? srow[key + u - slo] : 0.f;
         }
     };
-
-    float acc[kPrHeads][CPL];
+    // e / total, correctly rounded: q = e * (1 / total) is within two ulp, one
+    // residual step brings it within one, and a second (Markstein's theorem: a
+    // quotient within an ulp, the correctly rounded reciprocal and an exact
+    // residual) rounds it; residuals are exact from 2^-90 on (e <= 1 <= total).
+    // Tiny, infinite or NaN numerators and totals take the division.
+    auto weights = [&](int tile) {
+        float w[4];
+        bool plain = !(stotal < 0x1p30f);
 #pragma unroll
-    for (int hh = 0; hh < kPrHeads; ++hh)
+        for (int u = 0; u < 4; ++u) {
+            float q = ev[u] * srcp;
+            q = __builtin_fmaf(__builtin_fmaf(-q, stotal, ev[u]), srcp, q);
+            w[u] = __builtin_fmaf(__builtin_fmaf(-q, stotal, ev[u]), srcp, q);
+            plain = plain || !(ev[u] == 0.f || ev[u] >= 0x1p-90f);
+        }
+        if (__any(plain)) {
 #pragma unroll
-        for (int i = 0; i < CPL; ++i) acc[hh][i] = 0.f;
+            for (int u = 0; u < 4; ++u) w[u] = ev[u] / stotal;
+        }
+        float* d = at[tile & 1] + 4 * squad * NP + (spair ^ (4 * squad % NP));
+        if (stager) d[0] = w[0], d[NP] = w[1], d[2 * NP] = w[2], d[3 * NP] = w[3];
+    };
 
-    // one tile: keys j0 .. j0 + 31, four at a time; MASK: test each key
-    // against the lane's position
-    auto tile_sum = [&](const float* vbuf, const float* abuf, int j0, auto mask) {
+    const int hw = 2 * wave + (lane >> 5), p0 = PL * hw, cl = 4 * (lane & 31);
+    int lo[PL], hi[PL];
+#pragma unroll
+    for (int i = 0; i < PL; ++i) visible(p0 + i, lo[i], hi[i]);
+    float acc[PL][4];
+#pragma unroll
+    for (int i = 0; i < PL; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[i][e] = 0.f;
+    auto tile_sum = [&](int tile, auto mask) {
         constexpr bool M = decltype(mask)::value;
+        const float* vl = vt[tile & 1] + cl;
+        const float* al = at[tile & 1];
+        auto weight = [&](float (&w)[PL], int k) {
+            const float* p = al + k * NP + (p0 ^ (4 * (k / 4) % NP));
+            if constexpr (PL == 2) {
+                const float2 x = *reinterpret_cast<const float2*>(p);
+                w[0] = x.x, w[1] = x.y;
+            } else {
+                const float4 x = *reinterpret_cast<const float4*>(p);
+                w[0] = x.x, w[1] = x.y, w[2] = x.z, w[3] = x.w;
+            }
+        };
+        float wn[PL];  // the next key
+        float4 vn = *reinterpret_cast<const float4*>(vl);
+        weight(wn, 0);
 #pragma unroll
-        for (int kq = 0; kq < kPrKeys / 4; ++kq) {
-            float4 al[kPrHeads];
+        for (int k = 0; k < kPrKeys; ++k) {
+            const float v[4] = {vn.x, vn.y, vn.z, vn.w};
+            float w[PL];
 #pragma unroll
-            for (int hh = 0; hh < kPrHeads; ++hh) al[hh] = *reinterpret_cast<const float4*>(abuf + 4 * (kq * NP + hh * R + r));
+            for (int i = 0; i < PL; ++i) w[i] = wn[i];
+            if (k + 1 < kPrKeys) {
+                vn = *reinterpret_cast<const float4*>(vl + (k + 1) * kAttnDim);
+                weight(wn, k + 1);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            const int key = tile * kPrKeys + k;
 #pragma unroll
-            for (int kk = 0; kk < 4; ++kk) {
-                const float* vrow = vbuf + (4 * kq + kk) * kAttnDim + 32 * wave + CPL * cg;
-                float vv[CPL];
+            for (int i = 0; i < PL; ++i) {
+                const bool use = !M || (key >= lo[i] && key <= hi[i]);
 #pragma unroll
-                for (int i = 0; i < CPL; i += 4) {
-                    const float4 q = *reinterpret_cast<const float4*>(vrow + i);
-                    vv[i] = q.x, vv[i + 1] = q.y, vv[i + 2] = q.z, vv[i + 3] = q.w;
-                }
-                const bool use = !M || j0 + 4 * kq + kk <= my_pos;
-#pragma unroll
-                for (int hh = 0; hh < kPrHeads; ++hh) {
-                    const float w = kk == 0 ? al[hh].x : kk == 1 ? al[hh].y : kk == 2 ? al[hh].z : al[hh].w;
-#pragma unroll
-                    for (int i = 0; i < CPL; ++i) {
-                        const float sum = acc[hh][i] + w * vv[i];
-                        acc[hh][i] = M ? (use ? sum : acc[hh][i]) : sum;
-                    }
+                for (int e = 0; e < 4; ++e) {
+                    const float sum = acc[i][e] + w[i] * v[e];
+                    acc[i][e] = use ? sum : acc[i][e];
                 }
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
 
-    issue(0);
-    for (int tile = 0; tile < ntiles; ++tile) {
+    issue(tile0);
+    weights(tile0);
+    for (int tile = tile0; tile <= tile1; ++tile) {
         wait_vmcnt<0>();
         __syncthreads();  // the tile has landed everywhere; the other buffer's readers are done
-        if (tile + 1 < ntiles) issue(tile + 1);
-        const float* vbuf = vt[tile & 1];
-        const float* abuf = at[tile & 1];
-        if (tile < full_tiles)
-            tile_sum(vbuf, abuf, tile * kPrKeys, std::false_type{});
+        if (tile < tile1) issue(tile + 1);
+        if (tile * kPrKeys >= all_lo && tile * kPrKeys + kPrKeys - 1 <= all_hi)
+            tile_sum(tile, std::false_type{});
         else
-            tile_sum(vbuf, abuf, tile * kPrKeys, std::true_type{});
+            tile_sum(tile, std::true_type{});
+        if (tile < tile1) weights(tile + 1);
     }
 
-    // gate, Q8_0 block of each (row, head): 32 channels over the CG lanes of the row
+    // gate, Q8_0 blocks: 32 channels over eight lanes
     const int64_t width = int64_t(a.Hq) * DH;
     int8_t* qs = static_cast<int8_t*>(a.act_out);
     float* qd = reinterpret_cast<float*>(qs + int64_t(a.B) * width);
-    const int ch0 = part * kAttnDim + 32 * wave + CPL * cg;
 #pragma unroll
-    for (int hh = 0; hh < kPrHeads; ++hh) {
-        const int h = h0 + min(hh, nh - 1);
-        const float* gate = a.proj + int64_t(my_row) * a.proj_stride + int64_t(h) * 2 * DH + DH + ch0;
-        float out[CPL];
+    for (int i = 0; i < PL; ++i) {
+        const int pair = p0 + i, row = min(row0 + pair / hp, a.B - 1), h = h0 + min(pair % hp, nh - 1);
+        const float4 gate = *reinterpret_cast<const float4*>(a.proj + int64_t(row) * a.proj_stride + int64_t(h) * 2 * DH + DH + part * kAttnDim + cl);
+        const float out[4] = {acc[i][0] * sigmoid_f32(gate.x), acc[i][1] * sigmoid_f32(gate.y), acc[i][2] * sigmoid_f32(gate.z), acc[i][3] * sigmoid_f32(gate.w)};
         float amax = 0.f;
 #pragma unroll
-        for (int i = 0; i < CPL; ++i) {
-            out[i] = acc[hh][i] * sigmoid_f32(gate[i]);
-            amax = fmaxf(amax, fabsf(out[i]));
-        }
+        for (int e = 0; e < 4; ++e) amax = fmaxf(amax, fabsf(out[e]));
 #pragma unroll
-        for (int off = R; off < 64; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
+        for (int off = 1; off < 8; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off));
         const float d = amax / 127.f;
         const float id = d != 0.f ? 1.f / d : 0.f;
-        if (r < nrows && hh < nh) {
-            const int64_t idx = int64_t(my_row) * width + int64_t(h) * DH + ch0;
-            if (a.out_f32)
+        if (hi[i] >= 0) {
+            const int64_t o = int64_t(row) * width + int64_t(h) * DH + part * kAttnDim + cl;
+            if (a.out_f32) *reinterpret_cast<float4*>(a.out_f32 + o) = make_float4(out[0], out[1], out[2], out[3]);
+            uint32_t pk = 0;
 #pragma unroll
-                for (int i = 0; i < CPL; i += 4) *reinterpret_cast<float4*>(a.out_f32 + idx + i) = make_float4(out[i], out[i + 1], out[i + 2], out[i + 3]);
-            uint32_t pk[CPL / 4];
-#pragma unroll
-            for (int i = 0; i < CPL; i += 4) {
-                uint32_t w = 0;
-#pragma unroll
-                for (int u = 0; u < 4; ++u) w |= uint32_t(uint8_t(int8_t(int(roundf(out[i + u] * id))))) << (8 * u);
-                pk[i / 4] = w;
-            }
-#pragma unroll
-            for (int i = 0; i < CPL / 4; ++i) reinterpret_cast<uint32_t*>(qs + idx)[i] = pk[i];
-            if (cg == 0) qd[idx >> 5] = half_bits_to_f32(fp32_to_fp16_ref(d));
+            for (int e = 0; e < 4; ++e) pk |= uint32_t(uint8_t(int8_t(int(roundf(out[e] * id))))) << (8 * e);
+            *reinterpret_cast<uint32_t*>(qs + o) = pk;
+            if ((lane & 7) == 0) qd[o >> 5] = half_bits_to_f32(fp32_to_fp16_ref(d));
         }
     }
+}
+
+template <int DH, int PL>
+static void attn_pv_rows(const AttnDecodeArgs& a, unsigned blocks, hipStream_t s) {
+    const int R = kPrThreads / 32 * PL / rb_heads(a.Hq / a.Hkv);
+    hipLaunchKernelGGL((attn_pv_rows_kernel<DH, PL>), dim3(blocks, unsigned((a.B + R - 1) / R)), dim3(kPrThreads), 0, s, a);
+}
+
+// pair blocks of the weighted sum with PL pairs per lane
+static int64_t pv_row_blocks(const AttnDecodeArgs& a, int PL) {
+    const int group = a.Hq / a.Hkv, R = kPrThreads / 32 * PL / rb_heads(group);
+    return int64_t(a.Hkv) * rb_chunks(group) * (a.Dh / kAttnDim) * ((a.B + R - 1) / R);
+}
+
+// Which prefill chunks run in pair blocks: all but short ones under a sliding
+// window, where the per-row kernels' many workgroups are faster while the pair
+// blocks leave half the compute units without one (16 rows, window 512: 27 us
+// against 32; 128 rows 72 against 38).
+static bool attn_prefill_in_blocks(const AttnDecodeArgs& a) { return a.window == 0 || 2 * pv_row_blocks(a, 2) >= device_cus(); }
+
+template <int DH>
+static void attn_prefill_rows(const AttnDecodeArgs& a, hipStream_t s) {
+    const int group = a.Hq / a.Hkv, R = kRbPairs / rb_heads(group);
+    const int64_t cus = device_cus(), blocks = int64_t(a.Hkv) * rb_chunks(group), rows = (a.B + R - 1) / R;
+    hipLaunchKernelGGL(attn_prep_kernel<DH>, dim3(unsigned(a.Hq), unsigned(a.B)), dim3(DH), 0, s, a);
+    if (a.window == 0 && blocks * rows >= 2 * cus) {
+        // keys split over workgroups until there are eight per compute unit
+        const int64_t split = std::min<int64_t>((8 * cus + blocks * rows - 1) / (blocks * rows), (a.max_ctx + 255) / 256);
+        hipLaunchKernelGGL(attn_scores_rows_kernel<DH>, dim3(unsigned(blocks), unsigned(rows), unsigned(split)), dim3(256), 0, s, a);
+    } else {
+        // fewer rows, or windows (of which a 256-key tile covers much that is not
+        // seen): a lane per key and row (256 rows after 300: the call 127 us
+        // against 115; 1024 rows, window 512: 330 against 315)
+        const int64_t vis = a.window > 0 ? std::min<int64_t>(a.max_ctx, a.window) : a.max_ctx;
+        hipLaunchKernelGGL(attn_scores_kernel<DH>, dim3(unsigned(a.Hkv * ((group + kScoreHeads - 1) / kScoreHeads)), unsigned(std::min<int64_t>(kScoreTiles, (vis + 255) / 256)), unsigned(a.B)),
+                           dim3(256), 0, s, a);
+    }
+    hipLaunchKernelGGL(attn_softmax_rows_kernel, dim3(unsigned((int64_t(a.B) * a.Hq + kSrPairs - 1) / kSrPairs)), dim3(256), 0, s, a);
+    // four pairs a lane while that leaves two workgroups per compute unit, else
+    // two (512 rows of 128-wide heads: the call 140 us with four, 129 with two;
+    // 1024 rows: 303 and 343)
+    if (pv_row_blocks(a, 4) >= 2 * cus)
+        attn_pv_rows<DH, 4>(a, unsigned(blocks * (DH / kAttnDim)), s);
+    else
+        attn_pv_rows<DH, 2>(a, unsigned(blocks * (DH / kAttnDim)), s);
 }
 
 // ---- paged fp16 cache, split-K ------------------------------------------------------------
@@ -1952,16 +2240,16 @@ void attn_decode_wide(const AttnDecodeArgs& a, unsigned chunks, unsigned tiles, 
         hipLaunchKernelGGL(attn_softmax_regs_kernel<256>, dim3(unsigned(a.Hq), unsigned(a.B)), dim3(256), 0, s, a);
     else
         hipLaunchKernelGGL(attn_softmax_kernel, dim3(unsigned(a.Hq), unsigned(a.B)), dim3(seqsum::kThreads), 0, s, a);
-    if (a.shared_cache && a.window == 0 && a.max_ctx % 4 == 0) {  // a prefill chunk: the row-block weighted sum, per 128-channel part
-        hipLaunchKernelGGL((attn_pv_rows_kernel<kPrRows, DH>), dim3(chunks * (DH / kAttnDim), unsigned((a.B + kPrRows - 1) / kPrRows)), dim3(kPrThreads), 0, s, a);
-        return;
-    }
     hipLaunchKernelGGL(attn_pv_batch_kernel<DH>, dim3(unsigned(a.Hkv * ((group + kPvbHeads - 1) / kPvbHeads) * (DH / kPvbCh)), unsigned(a.B)), dim3(kPvbThreads), 0, s,
                        a);
 }
 }  // namespace
 
 void launch_attn_decode(const AttnDecodeArgs& a, hipStream_t s) {
+    if (a.shared_cache && attn_prefill_in_blocks(a)) {
+        a.Dh == 256 ? attn_prefill_rows<256>(a, s) : attn_prefill_rows<kAttnDim>(a, s);
+        return;
+    }
     const int64_t vis = a.window > 0 ? std::min<int64_t>(a.max_ctx, a.window) : a.max_ctx;
     const unsigned tiles = unsigned(std::min<int64_t>(kScoreTiles, (vis + 255) / 256));
     const int group = a.Hq / a.Hkv;
@@ -1977,13 +2265,6 @@ void launch_attn_decode(const AttnDecodeArgs& a, hipStream_t s) {
     } else {
         hipLaunchKernelGGL(attn_prep_kernel<kAttnDim>, dim3(unsigned(a.Hq), unsigned(a.B)), dim3(kAttnDim), 0, s, a);
         hipLaunchKernelGGL(attn_scores_kernel<kAttnDim>, dim3(chunks, tiles, unsigned(a.B)), dim3(256), 0, s, a);
-    }
-    // a prefill chunk (rows of one sequence, full causal visibility): the
-    // register softmax and the row-block weighted sum
-    if (a.shared_cache && a.window == 0 && a.max_ctx % 4 == 0) {
-        hipLaunchKernelGGL(attn_softmax_regs_kernel<256>, dim3(unsigned(a.Hq), unsigned(a.B)), dim3(256), 0, s, a);
-        hipLaunchKernelGGL((attn_pv_rows_kernel<kPrRows, kAttnDim>), dim3(unsigned(chunks), unsigned((a.B + kPrRows - 1) / kPrRows)), dim3(kPrThreads), 0, s, a);
-        return;
     }
     // the per-head pipeline while its workgroups fit the CUs (a deep ring, one
     // workgroup per CU) or fit them twice over (a shallower ring); for up to

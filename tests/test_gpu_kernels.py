@@ -712,6 +712,18 @@ def test_attn_prefill_rows_match_oracle(lib, M, p0, hq, hkv, max_ctx, window, dh
         assert blocks[b].tobytes() == oracle.quantize_row_q8_0(got[b]).tobytes(), f"row {b}"
 
 
+# the pair-block forms at the lines where they begin and in their odd shapes:
+# 513 rows (score blocks) with groups of 3 heads and a cache that ends inside a
+# score tile; 530 rows of 256-wide heads (four pairs a lane); groups of 1, 2
+# and 5 heads; a window whose scale of 1 spreads the scores so far that weights
+# underflow (the division beside the fast quotient), over a row stride that is
+# no multiple of 4; bit for bit, as the test above
+@pytest.mark.parametrize("M,p0,hq,hkv,max_ctx,window,dh", [(513, 0, 24, 8, 513, 0, 128), (530, 3, 32, 8, 535, 0, 256), (20, 5, 4, 4, 32, 0, 128), (21, 300, 8, 4, 323, 0, 128),
+                                                           (33, 7, 10, 2, 42, 0, 256), (130, 60, 32, 8, 191, 50, 128), (1, 30, 8, 2, 40, 0, 128)])
+def test_attn_prefill_pair_blocks_match_oracle(lib, M, p0, hq, hkv, max_ctx, window, dh):
+    test_attn_prefill_rows_match_oracle(lib, M, p0, hq, hkv, max_ctx, window, dh)
+
+
 @pytest.mark.parametrize("hq,window,page,dh", [(8, 0, 16, 128), (8, 50, 16, 128), (16, 0, 16, 128), (8, 0, 64, 128), (8, 50, 64, 128),
                                                 (8, 70, 64, 128), (16, 0, 64, 128), (8, 0, 64, 256), (8, 70, 64, 256), (16, 50, 64, 256)])
 def test_attn_paged_fp16_matches_oracle_over_fp16_kv(lib, hq, window, page, dh):
