@@ -730,29 +730,23 @@ namespace hero {
 // = row 4*(l/16)+r, column l%16.
 //
 // Workgroup: 256 lanes, a BM x 64 tile of Y; the four waves form a grid over
-// it (4 x 1 for BM >= 64: 32 or 16 rows x 64 columns each; 2 x 2 at BM = 32;
+// it (4 x 1 at BM = 64: 16 rows x 64 columns each; 2 x 2 at BM = 32;
 // 1 x 4 at BM = 16), so at the tall tiles a wave's operand and scale reads
 // serve two or four MFMAs each (unrolling a whole chunk of 8 blocks measured
 // slower: more registers, a worse schedule). K streams through shared memory
-// in chunks of KC blocks (gemm_kc: 4 at BM = 128, 8 below), tile rows padded
-// by 16 bytes (16 rows' 8-byte operand reads hit distinct banks); at BM = 128
-// the 4-block chunk halves the staging registers (117 instead of 204 VGPRs:
-// four waves per SIMD instead of two). The next chunk's bytes and scales are loaded into registers
+// in chunks of 8 blocks, tile rows padded by 16 bytes (16 rows' 8-byte operand
+// reads hit distinct banks). The next chunk's bytes and scales are loaded into registers
 // while the current chunk is computed (raw buffer loads sized to the tile, so
 // rows, blocks and scales past the edges read zeros without a branch), then
 // stored to shared memory between two barriers.
 // ---------------------------------------------------------------------------
 typedef int v4i_t __attribute__((ext_vector_type(4)));
 constexpr int kGemmBN = 64;
-// K blocks per shared-memory chunk: 4 at the 128-row tile (half the staging
-// registers: four waves per SIMD), 8 below (fewer barriers; at BM = 64 the
-// 4-block chunk measured 20% slower)
-template <int BM>
-constexpr int gemm_kc() { return BM >= 128 ? 4 : 8; }
+constexpr int kGemmKC = 8;  // K blocks per shared-memory chunk (4 measured 20% slower at BM = 64)
 
 template <int BM, int EPI>
 __global__ __launch_bounds__(256) void gemm_q8_kernel(const int8_t* __restrict__ wq, const uint16_t* __restrict__ wd, const int8_t* __restrict__ xq, const float* __restrict__ xd, float* __restrict__ y, const float* __restrict__ resid, int M, int N, int Npad, int K) {
-    constexpr int kGemmKC = gemm_kc<BM>(), kGemmRow = kGemmKC * 32 + 16;
+    constexpr int kGemmRow = kGemmKC * 32 + 16;
     __shared__ __align__(16) int8_t Xs[BM * kGemmRow];
     __shared__ __align__(16) int8_t Ws[kGemmBN * kGemmRow];
     __shared__ __align__(16) float dxs[kGemmKC][BM];  // [block][row]: a lane's 4 rows are one 16-byte read
@@ -887,6 +881,194 @@ __global__ __launch_bounds__(256) void gemm_q8_kernel(const int8_t* __restrict__
                 }
             }
         }
+}
+
+// ---------------------------------------------------------------------------
+// The same product for tall tiles, with the fp32 terms at three vector
+// instructions per output and block instead of four.
+//
+// A term is float(sumi) * (d_w * d_x), added in block order. Two of its parts
+// come from the matrix cores, whose int8 and fp16 forms run beside the vector
+// units:
+//  * the MFMA's addend is the bit pattern of 1.5 * 2^23, so the int32 result
+//    read as fp32 is 1.5 * 2^23 + sumi (|sumi| <= 2^19), and a subtraction
+//    gives float(sumi) exactly (an int-to-float conversion runs at half its rate);
+//  * d_w * d_x is a 32 x 32 fp16 outer product: both scales are fp16 values, so
+//    the fp32 product is exact (22 bits), as the reference's is.
+// Waves in pairs: a SIMD takes two waves' vector instructions side by side.
+//
+// Workgroup: 256 lanes, a tile of 64 rows x 128 columns, four waves as 2 x 2, each
+// 32 x 64 (128 x 64 tiles: 4% slower; 128 x 128: spills; 64 x 64: 30% slower; with
+// a second shared-memory buffer and one barrier a chunk: no faster). K streams through shared memory 4 blocks at a time as in
+// gemm_q8_kernel (blocks past the end read zeros: their terms are +0). Tile by
+// tile, the MFMAs of the next one are issued before the terms of this one.
+// Operand lanes (checked on the device): i8 32x32x32: A lane l row l % 32,
+// bytes 16 (l / 32) ..; f16 32x32x8: k 4 (l / 32) .. (only k = 0 is used); C
+// register v of lane l: row 8 (v / 4) + 4 (l / 32) + v % 4, column l % 32.
+//
+// Bound: those vector instructions (6.75 clocks of a SIMD per 64 outputs and
+// block); measured, quantizer
+// included, against gemm_q8_kernel with 128-row tiles: 1000 rows x 12288, K 4096
+// 204 -> 177 us, x 4096 97 -> 70, K 12288 x 4096 266 -> 186, 300 rows x 12288 113
+// -> 65. At 2.08 GHz (the clock drops under this load) a SIMD issues an instruction
+// every 4.5 clocks, half of what two waves could: they wait on the MFMAs' results.
+// ---------------------------------------------------------------------------
+typedef int v16i_t __attribute__((ext_vector_type(16)));
+typedef float v16s_t __attribute__((ext_vector_type(16)));
+typedef _Float16 v4h_t __attribute__((ext_vector_type(4)));
+constexpr int kMmKC = 4, kMmRow = kMmKC * 32 + 16;
+
+template <int EPI>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_q8_mm_kernel(
+    const int8_t* __restrict__ wq, const uint16_t* __restrict__ wd, const int8_t* __restrict__ xq, const float* __restrict__ xd, float* __restrict__ y,
+    const float* __restrict__ resid, int M, int N, int Npad, int K) {
+    constexpr int MT = 1, NT = 2, BM = 64 * MT, BN = 64 * NT;
+    __shared__ __align__(16) int8_t Xs[BM * kMmRow];
+    __shared__ __align__(16) int8_t Ws[BN * kMmRow];
+    __shared__ uint32_t dxs[kMmKC][BM], dws[kMmKC][BN];  // fp16 bits
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c32 = lane & 31, h = lane >> 5;
+    const int n0 = blockIdx.x * BN, m0 = blockIdx.y * BM;
+    const int nb = K >> 5;
+    const int mrows = min(BM, M - m0), nrows = min(BN, N - n0);
+    const __amdgpu_buffer_rsrc_t bx = buffer_of(xq + int64_t(m0) * K, uint32_t(mrows) * uint32_t(K));
+    const __amdgpu_buffer_rsrc_t bw = buffer_of(wq + int64_t(n0) * K, uint32_t(nrows) * uint32_t(K));
+    const __amdgpu_buffer_rsrc_t bdx = buffer_of(xd + int64_t(m0) * nb, uint32_t(mrows) * uint32_t(nb) * 4u);
+    const __amdgpu_buffer_rsrc_t bdw = buffer_of(wd + scale_index(n0, 0, nb), uint32_t((min(BN, Npad - n0) + 7) / 8) * uint32_t(nb) * 16u);
+    constexpr int XP = BM * 8 / 256, WP = BN * 8 / 256, DXP = BM * kMmKC / 256, DWP = BN * kMmKC / 256;
+    int4 xr[XP], wr[WP];
+    float dxr[DXP];
+    uint32_t dwr[DWP];
+    auto fetch = [&](int b0) {
+        const int kc = min(kMmKC, nb - b0);
+#pragma unroll
+        for (int q = 0; q < XP; ++q) {
+            const int e = tid + 256 * q, r = e / 8, c = e % 8;
+            xr[q] = load_b128(bx, c < 2 * kc ? uint32_t(r) * uint32_t(K) + uint32_t(b0) * 32u + uint32_t(c) * 16u : kOOB);
+        }
+#pragma unroll
+        for (int q = 0; q < WP; ++q) {
+            const int e = tid + 256 * q, r = e / 8, c = e % 8;
+            wr[q] = load_b128(bw, c < 2 * kc ? uint32_t(r) * uint32_t(K) + uint32_t(b0) * 32u + uint32_t(c) * 16u : kOOB);
+        }
+#pragma unroll
+        for (int q = 0; q < DXP; ++q) {
+            const int e = tid + 256 * q, r = e / kMmKC, bb = e % kMmKC;
+            dxr[q] = load_f32(bdx, bb < kc ? (uint32_t(r) * uint32_t(nb) + uint32_t(b0 + bb)) * 4u : kOOB);
+        }
+#pragma unroll
+        for (int q = 0; q < DWP; ++q) {
+            const int e = tid + 256 * q, bb = e / BN, c = e % BN;
+            const uint32_t off = (uint32_t(c >> 3) * uint32_t(nb) + uint32_t(b0 + bb)) * 16u + uint32_t(c & 7) * 2u;
+            dwr[q] = uint16_t(__builtin_amdgcn_raw_buffer_load_b16(bdw, bb < kc ? off : kOOB, 0, 0));
+        }
+    };
+    auto stage = [&]() {
+#pragma unroll
+        for (int q = 0; q < XP; ++q) {
+            const int e = tid + 256 * q;
+            *reinterpret_cast<int4*>(Xs + (e / 8) * kMmRow + (e % 8) * 16) = xr[q];
+        }
+#pragma unroll
+        for (int q = 0; q < WP; ++q) {
+            const int e = tid + 256 * q;
+            *reinterpret_cast<int4*>(Ws + (e / 8) * kMmRow + (e % 8) * 16) = wr[q];
+        }
+#pragma unroll
+        for (int q = 0; q < DXP; ++q) {
+            const int e = tid + 256 * q;
+            dxs[e % kMmKC][e / kMmKC] = __builtin_bit_cast(uint16_t, _Float16(dxr[q]));  // exact: an fp16 value
+        }
+#pragma unroll
+        for (int q = 0; q < DWP; ++q) {
+            const int e = tid + 256 * q;
+            dws[e / BN][e % BN] = dwr[q];
+        }
+    };
+
+    float acc[MT][NT][16];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+    v16i_t magic;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) magic[v] = 0x4B400000;
+    const uint32_t k0 = h ? 0u : 0xFFFFu;  // lanes that hold k = 0 of the outer product
+    const int8_t* xl = Xs + (32 * MT * (w >> 1) + c32) * kMmRow + 16 * h;
+    const int8_t* wl = Ws + (32 * NT * (w & 1) + c32) * kMmRow + 16 * h;
+    struct Ops {
+        v4b_t a[MT], b[NT];
+        uint32_t dx[MT], dw[NT];
+    };
+    auto operands = [&](Ops& o, int bb) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            o.a[i] = *reinterpret_cast<const v4b_t*>(xl + 32 * i * kMmRow + 32 * bb);
+            o.dx[i] = dxs[bb][32 * MT * (w >> 1) + 32 * i + c32];
+        }
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            o.b[j] = *reinterpret_cast<const v4b_t*>(wl + 32 * j * kMmRow + 32 * bb);
+            o.dw[j] = dws[bb][32 * NT * (w & 1) + 32 * j + c32];
+        }
+    };
+    struct Tile {
+        v16i_t sum;
+        v16s_t scale;
+    };
+    auto scale_op = [&](uint32_t d) { return __builtin_bit_cast(v4h_t, make_uint2(d & k0, 0u)); };
+    auto multiply = [&](const Ops& o, int i, int j) {
+        Tile t;
+        t.sum = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.a[i], o.b[j], magic, 0, 0, 0);
+        t.scale = __builtin_amdgcn_mfma_f32_32x32x8f16(scale_op(o.dx[i]), scale_op(o.dw[j]), v16s_t{}, 0, 0, 0);
+        return t;
+    };
+
+    fetch(0);
+    for (int b0 = 0; b0 < nb; b0 += kMmKC) {
+        stage();
+        __syncthreads();
+        if (b0 + kMmKC < nb) fetch(b0 + kMmKC);  // in flight during this chunk's compute
+        Ops cur, nxt;
+        operands(cur, 0);
+        Tile t = multiply(cur, 0, 0);
+#pragma unroll
+        for (int bb = 0; bb < kMmKC; ++bb) {
+            if (bb + 1 < kMmKC) operands(nxt, bb + 1);
+#pragma unroll
+            for (int ij = 0; ij < MT * NT; ++ij) {
+                Tile next;
+                if (ij + 1 < MT * NT)
+                    next = multiply(cur, (ij + 1) / NT, (ij + 1) % NT);
+                else if (bb + 1 < kMmKC)
+                    next = multiply(nxt, 0, 0);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[ij / NT][ij % NT][v] += (__int_as_float(t.sum[v]) - 12582912.f) * t.scale[v];
+                __builtin_amdgcn_sched_barrier(0);
+                t = next;
+            }
+            cur = nxt;
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int m = m0 + 32 * (MT * (w >> 1) + i) + 8 * (v >> 2) + 4 * h + (v & 3), n = n0 + 32 * (NT * (w & 1) + j) + c32;
+                if (m < M && n < N) {
+                    const int64_t o = int64_t(m) * N + n;
+                    if constexpr (EPI == kEpiResidual)
+                        y[o] = resid[o] + acc[i][j][v];
+                    else
+                        y[o] = acc[i][j][v];
+                }
+            }
 }
 
 // ---------------------------------------------------------------------------
@@ -1398,7 +1580,7 @@ int gemm_q8_plan(int64_t M, int64_t N, int64_t K) {
     // term work per CU is the same; more workgroups hide more latency)
     const int64_t tiles_n = (N + kGemmBN - 1) / kGemmBN, want = 2 * device_cus();
     auto grid_of = [&](int64_t bm) { return tiles_n * ((M + bm - 1) / bm); };
-    if (M > 64 && grid_of(128) >= want) return 128;
+    if (M > 64 && grid_of(128) >= want) return 128;  // gemm_q8_mm_kernel: as many tiles of 64 x 128
     if (M > 32 && grid_of(64) >= want) return 64;
     if (M > 16 && grid_of(32) >= want) return 32;
     return 16;
@@ -1490,7 +1672,12 @@ void launch_gemm_q8(const void* packed, const void* act, float* y, const float* 
             hipLaunchKernelGGL((gemm_q8_skinny_kernel<kEpiStore, NW>), dim3(grid_for(gemm_q8_skinny_kernel<kEpiStore, NW>, 64 * NW, smem)), dim3(64 * NW), smem, s, wq, wd, xq, xd, y, resid, int(M), int(N), Npad, int(K));
         break;
     }
-    case 128: gemm_dispatch<128>(epi, wq, wd, xq, xd, y, resid, int(M), int(N), Npad, int(K), s); break;
+    case 128: {
+        const dim3 grid(unsigned((N + 127) / 128), unsigned((M + 63) / 64));
+        hipLaunchKernelGGL(epi == kEpiResidual ? gemm_q8_mm_kernel<kEpiResidual> : gemm_q8_mm_kernel<kEpiStore>, grid, dim3(256), 0, s, wq, wd, xq, xd, y, resid, int(M), int(N),
+                           Npad, int(K));
+        break;
+    }
     case 64: gemm_dispatch<64>(epi, wq, wd, xq, xd, y, resid, int(M), int(N), Npad, int(K), s); break;
     case 32: gemm_dispatch<32>(epi, wq, wd, xq, xd, y, resid, int(M), int(N), Npad, int(K), s); break;
     default: gemm_dispatch<16>(epi, wq, wd, xq, xd, y, resid, int(M), int(N), Npad, int(K), s); break;

@@ -99,7 +99,7 @@ int hero_q8_0_gemm(const void* packed, const void* act, float* y, const float* r
  * per range of 16-row groups with the activation rows in shared memory), 4
  * (skinny, two or four waves per range of 16-row groups, one per 16
  * activation rows: 16 < m <= 64) or the tiled kernel's rows per tile (16, 32,
- * 64, 128). The choice depends on the
+ * 64; 128 stands for the form of large products, 64 rows by 128 columns). The choice depends on the
  * device's compute-unit count. No counterpart in the reference (its matmul
  * has one form, nm/src/quant_i8.hpp:430-474); lets tests show that every
  * form was checked. */

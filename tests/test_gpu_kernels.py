@@ -795,6 +795,41 @@ def test_attn_paged_fp16_matches_oracle_over_fp16_kv(lib, hq, window, page, dh):
     assert checked == 16
 
 
+# the form of large products (64 x 128 tiles, scale products on the matrix
+# cores): partial tiles both ways, K ends inside a 4-block chunk, scales from
+# fp16 subnormals to the largest (and zero), rows whose scale is subnormal, zero
+# or overflows to inf; every value the reference's, bit for bit (NaNs as NaNs)
+@pytest.mark.parametrize("m,n,k", [(129, 16390, 96), (300, 11000, 160), (65, 32800, 32)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_q8_0_gemm_large_form_matches_oracle_bitwise(lib, m, n, k, residual):
+    import ctypes
+
+    plan = ctypes.c_int32()
+    check(lib.hero_q8_0_gemm_plan(m, n, k, ctypes.byref(plan)))
+    assert plan.value == 128
+    rng = np.random.default_rng(m + n + k)
+    w = np.zeros((n, k // 32), oracle.BLOCK)
+    w["qs"] = rng.integers(-128, 128, (n, k // 32, 32), dtype=np.int8)
+    w["qs"][0] = -128
+    w["d"] = rng.integers(0, 0x7C00, (n, k // 32)).astype(np.uint16)  # every finite magnitude, evenly over the codes
+    w["d"][1] = 0
+    x = (rng.standard_normal((m, k)) * np.exp(rng.uniform(-16, 8, (m, 1)))).astype(np.float32)
+    x[3] = 0
+    x[5, :32] = 1e9  # scale past fp16: inf
+    r = rng.standard_normal((m, n)).astype(np.float32)
+    src = dev(w)
+    packed = empty(lib.hero_q8_0_packed_bytes(n, k))
+    check(lib.hero_q8_0_pack(ptr(src), ptr(packed), n, k, 0, n, stream()))
+    act, y, rd = quantize_dev(lib, x), empty(m * n * 4), dev(r)
+    check(lib.hero_q8_0_gemm(ptr(packed), ptr(act), ptr(y), ptr(rd) if residual else None, m, n, k, stream()))
+    got, want = host(y, np.float32, (m, n)), oracle.matmul(w, n, k, x)
+    if residual:
+        want = r + want
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.array_equal(bits(got)[~nan], bits(want)[~nan])
+
+
 # ---- K-quant weights (Q4_K / Q6_K against Q8_K activations) -------------------
 def kquant_weights(rng, wtype, n, k):
     """random GGUF Q4_K / Q6_K blocks: random quants and scales, sane fp16 d"""
