@@ -982,7 +982,7 @@ __global__ __launch_bounds__(kPvbThreads) void attn_pv_batch_kernel(AttnDecodeAr
     }
 }
 
-// ---- prefill over the shared cache: softmax and weighted sum by row blocks ------------------
+// ---- softmax in registers: batches of sequences, short windowed prefill chunks -----------------
 // The softmax of one (row, query head) for n <= 4096 visible keys with the
 // scores held in registers: lane t holds elements PT t .. PT t + PT - 1, the
 // max is order-free, e_j = exp(s_j - max) stays in registers, the total is the
@@ -990,7 +990,7 @@ __global__ __launch_bounds__(kPvbThreads) void attn_pv_batch_kernel(AttnDecodeAr
 // shared memory for its fallback) and alpha_j = e_j / total is written back:
 // one read and one write of the scores where attn_softmax_kernel makes three
 // reads and two writes. 256-lane workgroups (16 terms a lane) let eight run
-// per CU when there are thousands of rows, as in a prefill chunk. The host
+// per CU when there are many rows. The host
 // runs it for max_ctx % 4 == 0 (16-byte aligned rows); rows of more than 4096
 // keys take the chunked form.
 template <int NT>

@@ -497,6 +497,40 @@ def test_gdn_prefill_scan_tile_edges_match_oracle(lib, chunks):
     test_gdn_prefill_chunks_match_oracle(lib, 4, chunks)
 
 
+@pytest.mark.parametrize("T,W,hk,hv", [(261, 4, 16, 32), (256, 1, 32, 32), (519, 8, 8, 16)])
+def test_gdn_prefill_many_tokens_per_workgroup_equals_single(lib, T, W, hk, hv):
+    """Chunks long enough for eight tokens per prep / output workgroup (a partial
+    last group, windows of 1, 4 and 8) against the same tokens in chunks that run
+    one token per workgroup, which the oracle tests cover: outputs, Q8_0 blocks,
+    state and conv ring equal byte for byte."""
+    from hero_amd._lib import GdnDecodeArgs
+
+    rng = np.random.default_rng(T + W)
+    dk = 128
+    cc = 2 * hk * dk + hv * dk
+    stride = cc + hv * dk + 2 * hv
+    proj = (rng.standard_normal((T, stride)) * 0.7).astype(np.float32)
+    taps, dt = dev((rng.standard_normal((cc, W)) * 0.5).astype(np.float32)), dev((rng.standard_normal(hv) * 0.1).astype(np.float32))
+    decay, gamma = dev((-np.exp(rng.standard_normal(hv) * 0.5)).astype(np.float32)), dev((1 + 0.1 * rng.standard_normal(dk)).astype(np.float32))
+    h0, s0 = rng.standard_normal((W, cc)).astype(np.float32), (rng.standard_normal((hv, dk, dk)) * 0.1).astype(np.float32)
+    wbytes = lib.hero_gdn_prefill_work_bytes(T, hk, hv)
+    work, width, res = empty(wbytes), hv * dk, []
+    for step in (T, 100):
+        hist, state, outs, blocks = dev(h0), dev(s0), [], []
+        for t in range(0, T, step):
+            n = min(step, T - t)
+            d_proj, d_pos = dev(proj[t:t + n]), dev(np.array([W + t], np.int32))
+            act, out = empty(lib.hero_q8_0_act_bytes(n, width)), empty(n * width * 4)
+            a = GdnDecodeArgs(ptr(d_proj), stride, cc, cc + width, cc + width + hv, ptr(taps), ptr(hist), ptr(state), ptr(dt), ptr(decay), ptr(gamma),
+                              np.float32(1e-6), ptr(d_pos), ptr(act), ptr(out), n, hk, hv, dk, dk, W)
+            check(lib.hero_gdn_prefill(a, ptr(work), wbytes, stream()))
+            outs.append(host(out, np.uint32, (n, width)))
+            blocks.append(act_to_blocks(host(act, np.uint8)[: n * width + n * width // 32 * 4], n, width))
+        res.append((np.concatenate(outs), np.concatenate(blocks), host(state, np.uint32).copy(), host(hist, np.uint32).copy()))
+    for i, what in enumerate(("output", "quantized output", "state", "ring")):
+        assert res[0][i].tobytes() == res[1][i].tobytes(), what
+
+
 @pytest.mark.parametrize("T,hk,hv", [(70, 2, 4), (300, 4, 4)])
 def test_gdn_chunked_prefill_matches_serial(lib, T, hk, hv):
     """The chunked (WY) delta-net prefill against the token-serial one (which
