@@ -688,6 +688,9 @@ __global__ __launch_bounds__(kGdnDim) void gdn_prep_kernel(GdnDecodeArgs a, void
 // in shared memory, with the same lanes and rows but lane r at token (step - r):
 // there all sixteen lanes' sums count, each its own token's. These waves also
 // stage the inputs.
+// Both groups of waves start from the state in memory, and the first one writes
+// it back: with 8 tokens or fewer before the first tile's barrier. So every wave
+// has its copy before the barrier that precedes the first tile.
 //
 // Bound: the prediction chain, 128 dependent adds and 15 shifts with their wait
 // states (~700 clocks of a token). Measured: 1024 tokens, 32 heads 785 -> 395 us
@@ -759,25 +762,28 @@ __global__ __launch_bounds__(512) void gdn_scan_cols_kernel(GdnDecodeArgs a, voi
     };
 
     const int phases = (T + 15 + kScTile - 1) / kScTile + 1;  // the outputs end 15 steps and a tile after the predictions
+    float col[8];  // S[8 r + m][column], for waves 4-7 at the token the lane has reached
+#pragma unroll
+    for (int m = 0; m < 8; ++m) col[m] = S[int64_t(8 * r + m) * kGdnDim];
     if (wave >= 4) {
         load(0);
         store(0);
         load(1);
         store(1);
-        load(2);
     }
+#pragma unroll
+    for (int m = 0; m < 8; ++m) asm volatile("" : "+v"(col[m]));  // the reads have returned: waves 0-3 overwrite the state past the barrier
+    if (wave >= 4) load(2);
     __syncthreads();
 
     if (wave < 4) {
         __builtin_amdgcn_s_setprio(3);
-        float col[8], kc[8];  // S[8 r + m][column], k[8 r + m]
+        float kc[8];  // k[8 r + m]
         auto keys = [&](int t, float (&k)[8]) {
             const float4* p = reinterpret_cast<const float4*>(sh.k[t & kMask] + 8 * r);
             const float4 x = p[0], y = p[1];
             k[0] = x.x, k[1] = x.y, k[2] = x.z, k[3] = x.w, k[4] = y.x, k[5] = y.y, k[6] = y.z, k[7] = y.w;
         };
-#pragma unroll
-        for (int m = 0; m < 8; ++m) col[m] = S[int64_t(8 * r + m) * kGdnDim];
         // token 0: decay and prediction chain (nm/src/recurrent.hpp:152-160)
         keys(0, kc);
         float pred;
@@ -827,9 +833,6 @@ __global__ __launch_bounds__(512) void gdn_scan_cols_kernel(GdnDecodeArgs a, voi
             __syncthreads();
         }
     } else {
-        float col[8];  // S[8 r + i][column] at this lane's token
-#pragma unroll
-        for (int i = 0; i < 8; ++i) col[i] = S[int64_t(8 * r + i) * kGdnDim];
         float acc = 0.f;
         for (int j = 0; j < phases; ++j) {
             store(j + 2);

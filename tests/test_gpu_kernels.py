@@ -497,6 +497,38 @@ def test_gdn_prefill_scan_tile_edges_match_oracle(lib, chunks):
     test_gdn_prefill_chunks_match_oracle(lib, 4, chunks)
 
 
+# chunks that end within the scan's first 8-token tile write the state back while
+# that tile is still worked on, so the waves that form the outputs must have read
+# it before (9 tokens: the first length that a barrier separates). A workgroup on
+# every compute unit, from a state that is not zero.
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 6, 7, 8, 9])
+def test_gdn_prefill_of_one_tile_equals_decode_steps(lib, T):
+    from hero_amd._lib import GdnDecodeArgs
+
+    hk, hv, dk, W = 16, 32, 128, 4
+    rng = np.random.default_rng(70 + T)
+    cc, width = 2 * hk * dk + hv * dk, hv * dk
+    stride = cc + width + 2 * hv
+    proj = (rng.standard_normal((T, stride)) * 0.7).astype(np.float32)
+    taps, dt = dev((rng.standard_normal((cc, W)) * 0.5).astype(np.float32)), dev((rng.standard_normal(hv) * 0.1).astype(np.float32))
+    decay, gamma = dev((-np.exp(rng.standard_normal(hv) * 0.5)).astype(np.float32)), dev((1 + 0.1 * rng.standard_normal(dk)).astype(np.float32))
+    h0, s0 = rng.standard_normal((W, cc)).astype(np.float32), (rng.standard_normal((hv, dk, dk)) * 0.1).astype(np.float32)
+    wbytes = lib.hero_gdn_prefill_work_bytes(T, hk, hv)
+    work, res = empty(wbytes), []
+    for step in (T, 1):
+        hist, state, outs = dev(h0), dev(s0), []
+        for t in range(0, T, step):
+            d_proj, d_pos = dev(proj[t:t + step]), dev(np.array([W + t], np.int32))
+            act, out = empty(lib.hero_q8_0_act_bytes(step, width)), empty(step * width * 4)
+            a = GdnDecodeArgs(ptr(d_proj), stride, cc, cc + width, cc + width + hv, ptr(taps), ptr(hist), ptr(state), ptr(dt), ptr(decay), ptr(gamma),
+                              np.float32(1e-6), ptr(d_pos), ptr(act), ptr(out), step, hk, hv, dk, dk, W)
+            check(lib.hero_gdn_prefill(a, ptr(work), wbytes, stream()) if len(res) == 0 else lib.hero_gdn_decode(a, stream()))
+            outs.append(host(out, np.uint32, (step, width)))
+        res.append((np.concatenate(outs), host(state, np.uint32).copy(), host(hist, np.uint32).copy()))
+    for i, what in enumerate(("output", "state", "ring")):
+        assert np.array_equal(res[0][i], res[1][i]), what
+
+
 @pytest.mark.parametrize("T,W,hk,hv", [(261, 4, 16, 32), (256, 1, 32, 32), (519, 8, 8, 16)])
 def test_gdn_prefill_many_tokens_per_workgroup_equals_single(lib, T, W, hk, hv):
     """Chunks long enough for eight tokens per prep / output workgroup (a partial
