@@ -37,6 +37,7 @@ inline int64_t act_q8_bytes(int64_t M, int64_t K) { return M * K + M * (K / 32) 
 int64_t act_q8_K_bytes(int64_t m, int64_t k);
 int64_t kquant_packed_bytes(int type, int64_t N, int64_t K);
 int kquant_max_k(int type);  // 65536 (Q4_K, Q6_K), 16384 (Q5_K)
+int kquant_gemm_plan(int type, int64_t M, int64_t N, int64_t K);  // which form a product takes (hero_kquant_gemm_plan)
 void launch_kquant_pack(int type, const void* gguf, void* packed, int64_t N, int64_t K, hipStream_t s);
 void launch_quantize_q8_K(const float* x, void* act, int64_t M, int64_t K, hipStream_t s);
 // y[m * ldy + n] (+= resid[m * ldy + n], added after the product)

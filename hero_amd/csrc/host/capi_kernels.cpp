@@ -155,6 +155,16 @@ int hero_q5_K_gemm(const void* w, const float* x, float* y, int64_t m, int64_t n
     });
 }
 
+int hero_kquant_gemm_plan(int32_t type, int64_t m, int64_t n, int64_t k, int32_t* kernel) {
+    return guard([&] {
+        require(type == 12 || type == 13 || type == 14, "type must be 12 (Q4_K), 13 (Q5_K) or 14 (Q6_K)");
+        check_kquant_shape(type, n, k);
+        require(m > 0 && m <= (int64_t(1) << 31) / (k / 256), "m out of range");
+        require(kernel, "null pointer");
+        *kernel = kquant_gemm_plan(type, m, n, k);
+    });
+}
+
 int hero_kquant_dequant_rows(int32_t type, const void* w, int64_t n, int64_t k, const int32_t* ids, int64_t n_ids, float* out, void* stream) {
     return guard([&] {
         require(type == 12 || type == 13 || type == 14, "type must be 12 (Q4_K), 13 (Q5_K) or 14 (Q6_K)");

@@ -518,7 +518,7 @@ __global__ __launch_bounds__(kMmThreads) void kq_mm_kernel(const uint8_t* __rest
     constexpr int XC = BM * 16, WC = BN * U;  // 16-byte chunks of x and of the weights
     constexpr int XI = (XC + kMmThreads - 1) / kMmThreads, WI = (WC + kMmThreads - 1) / kMmThreads;
     const int R = kq_rows_per_tile(K), wpt = kq_waves_per_tile(K);
-    // chunk indices fit 32 bits: the launcher checks
+    // chunk indices fit 32 bits: kq_form() looks at the weights, the launcher slices the activation rows
     uint32_t xrow[XI];   // chunk tid % 16 of the row, super-block 0
     uint32_t wslot[WI];  // slot of super-block 0 of the chunk's row
 #pragma unroll
@@ -1169,37 +1169,47 @@ static void kq_mm(const uint8_t* w, const uint8_t* act, const uint32_t* xt, floa
                        int(tm), int(tn));
 }
 
+// The form of a Q4_K / Q6_K product: 1 the lane-per-block form, 32 or 64 the
+// matrix-core form with tiles of that many rows either way.
+static int kq_form(int type, int64_t M, int64_t N, int64_t K) {
+    // kq_mm_kernel's weight chunk indices are 32 bits; kq_gemm_kernel's are 64
+    // (477M super-blocks of Q4_K, 330M of Q6_K: 69 GB)
+    if (M == 1 || kq_slots(N, K) * kq_chunks(type) > int64_t(UINT32_MAX)) return 1;
+    // Which form, by estimates in microseconds (with the quantizer, fitted to
+    // M 2 .. 48, N 1000 .. 12288, K 1024 .. 12288): the lane-per-block form
+    // costs per pass of R weight rows x 4 activation rows on a compute unit,
+    // the matrix-core form per round of one 32 x 32 tile a compute unit (a
+    // 64 x 64 tile costs two) and super-block. Measured, former and matrix-core
+    // form: Q4_K 4096 x 4096: 12 rows 16.3 / 19.7, 16 rows 22.9 / 19.9, 48 rows
+    // 44.8 / 20.8; 1000 x 12288, 16 rows 26.7 / 44.3; Q6_K 4096 x 4096: 8 rows
+    // 18.2 / 19.4, 12 rows 27.2 / 21.6; 4096 x 12288, 9 rows 68.7 / 50.3.
+    const int nb = int(K / 256);
+    const int64_t cus = device_cus();
+    auto rounds = [&](int64_t t) { return ((M + t - 1) / t * ((N + t - 1) / t) + cus - 1) / cus; };
+    const int64_t small = rounds(32), large = rounds(64), R = kq_rows_per_tile(K);
+    const double passes = double((N + R - 1) / R) * double(M) / (4.0 * double(cus)), over = std::max(0, nb - 32);
+    const double lanes = type == 12 ? 9 + (3 + 0.1 * over) * passes : 10 + (5.2 + 0.06 * over) * passes;
+    const double tiles = (6 + (type == 12 ? 0.83 : 0.92) * nb) * (0.23 + 0.77 * double(std::min(small, 2 * large)));
+    if (tiles > lanes) return 1;
+    // the small tile takes about half the large one's time for a quarter of its
+    // outputs (Q4_K N 4096, K 4096: 64 rows 21 and 33 us, 509 rows 98 and 63 us)
+    return small <= 2 * large ? 32 : 64;
+}
+
 void launch_kquant_gemm_ld(int type, const void* w, const void* act, float* y, const float* resid, int64_t M, int64_t N, int64_t K, int64_t ldy,
                            hipStream_t s) {
     const int nb = int(K / 256);
     const auto* wb = static_cast<const uint8_t*>(w);
     const auto* ab = static_cast<const uint8_t*>(act);
     const uint32_t* xt = regrouped_of(act, M * nb);
-    if (M > 1) {
-        // Which form, by estimates in microseconds (with the quantizer, fitted to
-        // M 2 .. 48, N 1000 .. 12288, K 1024 .. 12288): the lane-per-block form
-        // costs per pass of R weight rows x 4 activation rows on a compute unit,
-        // the matrix-core form per round of one 32 x 32 tile a compute unit (a
-        // 64 x 64 tile costs two) and super-block. Measured, former and matrix-core
-        // form: Q4_K 4096 x 4096: 12 rows 16.3 / 19.7, 16 rows 22.9 / 19.9, 48 rows
-        // 44.8 / 20.8; 1000 x 12288, 16 rows 26.7 / 44.3; Q6_K 4096 x 4096: 8 rows
-        // 18.2 / 19.4, 12 rows 27.2 / 21.6; 4096 x 12288, 9 rows 68.7 / 50.3.
-        const int64_t cus = device_cus();
-        auto rounds = [&](int64_t t) { return ((M + t - 1) / t * ((N + t - 1) / t) + cus - 1) / cus; };
-        const int64_t small = rounds(32), large = rounds(64), R = kq_rows_per_tile(K);
-        const double passes = double((N + R - 1) / R) * double(M) / (4.0 * double(cus)), over = std::max(0, nb - 32);
-        const double lanes = type == 12 ? 9 + (3 + 0.1 * over) * passes : 10 + (5.2 + 0.06 * over) * passes;
-        const double tiles = (6 + (type == 12 ? 0.83 : 0.92) * nb) * (0.23 + 0.77 * double(std::min(small, 2 * large)));
-        if (tiles <= lanes) {
-            // the small tile takes about half the large one's time for a quarter
-            // of its outputs (Q4_K N 4096, K 4096: 64 rows 21 and 33 us, 509 rows
-            // 98 and 63 us); rows go in slices whose chunk indices fit 32 bits
-            auto run = small <= 2 * large ? (type == 12 ? kq_mm<12, 1, 1> : kq_mm<14, 1, 1>) : (type == 12 ? kq_mm<12, 2, 2> : kq_mm<14, 2, 2>);
-            const int64_t slice = int64_t(1) << 20;
-            for (int64_t r0 = 0; r0 < M; r0 += slice)
-                run(wb, ab + r0 * nb * kQ8KBytes, xt + r0 * nb * 64, y + r0 * ldy, resid ? resid + r0 * ldy : nullptr, std::min(slice, M - r0), N, K, ldy, s);
-            return;
-        }
+    const int form = kq_form(type, M, N, K);
+    if (form != 1) {
+        // rows go in slices whose chunk indices fit 32 bits
+        auto run = form == 32 ? (type == 12 ? kq_mm<12, 1, 1> : kq_mm<14, 1, 1>) : (type == 12 ? kq_mm<12, 2, 2> : kq_mm<14, 2, 2>);
+        const int64_t slice = int64_t(1) << 20;
+        for (int64_t r0 = 0; r0 < M; r0 += slice)
+            run(wb, ab + r0 * nb * kQ8KBytes, xt + r0 * nb * 64, y + r0 * ldy, resid ? resid + r0 * ldy : nullptr, std::min(slice, M - r0), N, K, ldy, s);
+        return;
     }
     int R, per;
     kq_plan(M, N, K, kKqTile, &R, &per);
@@ -1219,36 +1229,47 @@ void launch_kquant_gemm(int type, const void* w, const void* act, float* y, int6
     launch_kquant_gemm_ld(type, w, act, y, nullptr, M, N, K, N, s);
 }
 
-void launch_q5k_gemm(const void* w, const float* x, int64_t ldx, float* y, const float* resid, int64_t M, int64_t N, int64_t K, int64_t ldy, hipStream_t s) {
-    // activation rows per pass: shared memory holds TILE rows of K floats (<= 64 KiB)
-    const int tile = M == 1 ? 1 : K <= 4096 ? 4 : K <= 8192 ? 2 : 1;
-    int R, per;
-    kq_plan(M, N, K, tile, &R, &per);
-    // Several rows: the matrix-core form unless the lane-per-block form's
+// activation rows per pass of the lane-per-block form: shared memory holds as many rows of K floats (<= 64 KiB)
+static int q5k_tile(int64_t M, int64_t K) { return M == 1 ? 1 : K <= 4096 ? 4 : K <= 8192 ? 2 : 1; }
+
+// The form of a Q5_K product: 1 the lane-per-block form, 4 or 16 the
+// outer-product form with that many activation rows per tile.
+static int q5k_form(int64_t M, int64_t N, int64_t K) {
+    // Several rows: the outer-product form unless the lane-per-block form's
     // workgroup passes (one per R weight rows and tile activation rows; about 8,
     // 6.6 and 5 us each on a compute unit, at least 13) cost less than its 4-row
     // tiles (about 3 + 1.2 us per super-block of a row), both in microseconds.
     // Measured, former and this form: K 4096 x 4096 rows: 8 rows 19.4 / 22.1 us,
     // 10 rows 35.4 / 22.7; K 1024 x 1000, 2 rows: 12.8 / 9.4; K 8192 x 4096, 4
     // rows 27.3 / 39.8, 8 rows 53.2 / 41.1; K 12288 x 4096, 2 rows 45 / 62, 4 rows 80 / 61.
-    if (M > 1) {
-        const int64_t cus = device_cus(), nb = K / 256;
-        auto rounds = [&](int64_t rows, int64_t cols) { return ((M + rows - 1) / rows * ((N + cols - 1) / cols) + cus - 1) / cus; };
-        const double lanes = std::max(13.0, double(rounds(tile, R)) * (tile == 4 ? 8.0 : tile == 2 ? 6.6 : 5.0));
-        if (double(rounds(4, 64)) * (3.0 + 1.2 * double(nb)) < lanes) {
-            // 16-row tiles take three times a 4-row tile's time once the compute
-            // units are full (47 and 15.5 us at K 4096)
-            const int rows = 3 * rounds(16, 64) < rounds(4, 64) ? 16 : 4;
-            const int64_t slice = int64_t(65535) * rows;  // grid.y
-            for (int64_t r0 = 0; r0 < M; r0 += slice) {
-                const int64_t part = std::min(slice, M - r0);
-                hipLaunchKernelGGL(rows == 16 ? q5k_mm_kernel<16> : q5k_mm_kernel<4>, dim3(unsigned((N + 63) / 64), unsigned((part + rows - 1) / rows)),
-                                   dim3(64 * kQ5Waves), q5k_mm_shared(rows), s, static_cast<const uint8_t*>(w), x + r0 * ldx, ldx, y + r0 * ldy,
-                                   resid ? resid + r0 * ldy : nullptr, part, N, int(K), ldy);
-            }
-            return;
+    if (M == 1) return 1;
+    const int64_t cus = device_cus(), nb = K / 256;
+    const int tile = q5k_tile(M, K);
+    auto rounds = [&](int64_t rows, int64_t cols) { return ((M + rows - 1) / rows * ((N + cols - 1) / cols) + cus - 1) / cus; };
+    const double lanes = std::max(13.0, double(rounds(tile, kq_rows_per_tile(K))) * (tile == 4 ? 8.0 : tile == 2 ? 6.6 : 5.0));
+    if (double(rounds(4, 64)) * (3.0 + 1.2 * double(nb)) >= lanes) return 1;
+    // 16-row tiles take three times a 4-row tile's time once the compute units
+    // are full (47 and 15.5 us at K 4096)
+    return 3 * rounds(16, 64) < rounds(4, 64) ? 16 : 4;
+}
+
+int kquant_gemm_plan(int type, int64_t M, int64_t N, int64_t K) { return type == 13 ? q5k_form(M, N, K) : kq_form(type, M, N, K); }
+
+void launch_q5k_gemm(const void* w, const float* x, int64_t ldx, float* y, const float* resid, int64_t M, int64_t N, int64_t K, int64_t ldy, hipStream_t s) {
+    const int rows = q5k_form(M, N, K);
+    if (rows != 1) {
+        const int64_t slice = int64_t(65535) * rows;  // grid.y
+        for (int64_t r0 = 0; r0 < M; r0 += slice) {
+            const int64_t part = std::min(slice, M - r0);
+            hipLaunchKernelGGL(rows == 16 ? q5k_mm_kernel<16> : q5k_mm_kernel<4>, dim3(unsigned((N + 63) / 64), unsigned((part + rows - 1) / rows)),
+                               dim3(64 * kQ5Waves), q5k_mm_shared(rows), s, static_cast<const uint8_t*>(w), x + r0 * ldx, ldx, y + r0 * ldy,
+                               resid ? resid + r0 * ldy : nullptr, part, N, int(K), ldy);
         }
+        return;
     }
+    const int tile = q5k_tile(M, K);
+    int R, per;
+    kq_plan(M, N, K, tile, &R, &per);
     const dim3 grid(unsigned((N + R - 1) / R), unsigned((M + per - 1) / per));
     const size_t lds = size_t(tile) * K * 4;  // <= 64 KiB
     const auto* wb = static_cast<const uint8_t*>(w);

@@ -159,6 +159,11 @@ int hero_argmax_noalloc(const float* logits, int64_t m, int64_t n, int32_t* out,
  * hero_kquant_dequant_rows is Weight::dequant_row / gather_rows
  * (nm/src/quant.hpp:464-480) on a packed tensor: out[t][k] = row ids[t] (device
  * ids; an id outside [0, n) gives a row of zeros).
+ * hero_kquant_gemm_plan tells which kernel a product of m rows runs on the
+ * current device, without running it: *kernel = 1 (a lane per super-block) or
+ * the rows per tile of the matrix-core form: 32 or 64 (Q4_K, Q6_K), 4 or 16
+ * (Q5_K). As hero_q8_0_gemm_plan, it lets tests show that every form was
+ * checked; results do not depend on it.
  * k: a multiple of 256, at most 65536 (16384 for Q5_K). */
 int64_t hero_q8_K_act_bytes(int64_t m, int64_t k);
 int hero_q8_K_quantize(const float* x, void* act, int64_t m, int64_t k, void* stream);
@@ -166,6 +171,7 @@ int64_t hero_kquant_packed_bytes(int32_t type, int64_t n, int64_t k);
 int hero_kquant_pack(int32_t type, const void* gguf, void* packed, int64_t n, int64_t k, void* stream);
 int hero_kquant_gemm(int32_t type, const void* w, const void* act, float* y, int64_t m, int64_t n, int64_t k, void* stream);
 int hero_q5_K_gemm(const void* w, const float* x, float* y, int64_t m, int64_t n, int64_t k, void* stream);
+int hero_kquant_gemm_plan(int32_t type, int64_t m, int64_t n, int64_t k, int32_t* kernel);
 int hero_kquant_dequant_rows(int32_t type, const void* w, int64_t n, int64_t k, const int32_t* ids, int64_t n_ids, float* out, void* stream);
 
 /* Logits::sample with temp > 0 (nm/src/logits.hpp:71-105) on one row of v

@@ -72,6 +72,23 @@ def test_kquant_argument_errors_are_reported_before_any_launch():
     assert lib.hero_kquant_packed_bytes(8, 3, 512) == -1
 
 
+# the matrix-core forms index a weight's 16-byte chunks (9 of a Q4_K super-block,
+# 13 of a Q6_K one) with 32 bits: at k 4096 the last such matrix has
+# (2^32 - 1) // (16 * chunks) rows, 16 to a packed tile
+@pytest.mark.parametrize("wtype,chunks", [(12, 9), (14, 13)])
+@pytest.mark.parametrize("m,tile", [(16, 32), (256, 64)])
+def test_kquant_products_past_32_bit_chunk_indices_take_the_64_bit_form(wtype, chunks, m, tile):
+    def plan(n):
+        kernel = ctypes.c_int32()
+        assert _lib.lib.hero_kquant_gemm_plan(wtype, m, n, 4096, ctypes.byref(kernel)) == _lib.HERO_OK
+        return kernel.value
+
+    last = ((1 << 32) - 1) // (16 * chunks) // 16 * 16
+    assert plan(last) == tile
+    assert plan(last + 1) == 1  # one more packed tile
+    assert plan((1 << 31) // 16) == 1
+
+
 def test_size_helpers():
     assert _lib.lib.hero_q8_0_packed_bytes(4096, 4096) == 4096 * 4096 * 34 // 32
     assert _lib.lib.hero_q8_0_act_bytes(2, 1024) == 2 * 1024 + 2 * 32 * 4
