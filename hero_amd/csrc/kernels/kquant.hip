@@ -1169,6 +1169,17 @@ static void kq_mm(const uint8_t* w, const uint8_t* act, const uint32_t* xt, floa
                        int(tm), int(tn));
 }
 
+// Activation rows of one launch of kq_mm_kernel: 2^20 for its 32-bit activation
+// chunk indices, fewer where N is so large that the grid would pass 2^32 - 1
+// lanes (0: not even one tile of rows fits).
+constexpr int64_t kq_slice_rows(int64_t N, int64_t tile) {
+    const int64_t columns = ((N + tile - 1) / tile + 7) / 8 * 8, workgroups = ((int64_t(1) << 32) - 1) / kMmThreads;
+    return std::min(int64_t(1) << 20, workgroups / columns * tile);
+}
+static_assert(kq_slice_rows(32768 - 512, 64) == 1 << 20);  // 504 tile columns x 16384
+static_assert(kq_slice_rows(32768, 64) == (1 << 20) - 64);  // 512 x 16384 workgroups of 512 lanes are 2^32
+static_assert(kq_slice_rows((int64_t(1) << 32) / 9, 64) == 64 && kq_slice_rows(int64_t(1) << 28, 32) == 0);
+
 // The form of a Q4_K / Q6_K product: 1 the lane-per-block form, 32 or 64 the
 // matrix-core form with tiles of that many rows either way.
 static int kq_form(int type, int64_t M, int64_t N, int64_t K) {
@@ -1193,7 +1204,8 @@ static int kq_form(int type, int64_t M, int64_t N, int64_t K) {
     if (tiles > lanes) return 1;
     // the small tile takes about half the large one's time for a quarter of its
     // outputs (Q4_K N 4096, K 4096: 64 rows 21 and 33 us, 509 rows 98 and 63 us)
-    return small <= 2 * large ? 32 : 64;
+    const int tile = small <= 2 * large ? 32 : 64;
+    return kq_slice_rows(N, tile) > 0 ? tile : 1;
 }
 
 void launch_kquant_gemm_ld(int type, const void* w, const void* act, float* y, const float* resid, int64_t M, int64_t N, int64_t K, int64_t ldy,
@@ -1204,9 +1216,8 @@ void launch_kquant_gemm_ld(int type, const void* w, const void* act, float* y, c
     const uint32_t* xt = regrouped_of(act, M * nb);
     const int form = kq_form(type, M, N, K);
     if (form != 1) {
-        // rows go in slices whose chunk indices fit 32 bits
         auto run = form == 32 ? (type == 12 ? kq_mm<12, 1, 1> : kq_mm<14, 1, 1>) : (type == 12 ? kq_mm<12, 2, 2> : kq_mm<14, 2, 2>);
-        const int64_t slice = int64_t(1) << 20;
+        const int64_t slice = kq_slice_rows(N, form);
         for (int64_t r0 = 0; r0 < M; r0 += slice)
             run(wb, ab + r0 * nb * kQ8KBytes, xt + r0 * nb * 64, y + r0 * ldy, resid ? resid + r0 * ldy : nullptr, std::min(slice, M - r0), N, K, ldy, s);
         return;
