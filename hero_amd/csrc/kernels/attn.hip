@@ -1082,6 +1082,15 @@ __global__ __launch_bounds__(NT) void attn_softmax_regs_kernel(AttnDecodeArgs a)
 // side by side.
 constexpr int kRbPairs = 32;  // pairs of a score block
 
+// 16 bytes at any float's address: proj_stride may be odd, and of the prefill's
+// buffers only v_cache and act_out are read or written in wider pieces
+__device__ __forceinline__ float4 load_f4(const float* p) {
+    float4 v;
+    __builtin_memcpy(&v, p, 16);
+    return v;
+}
+__device__ __forceinline__ void store_f4(float* p, const float4& v) { __builtin_memcpy(p, &v, 16); }
+
 // query heads of a block (a power of two) and blocks per K/V group
 __host__ __device__ inline int rb_heads(int group) { return group >= 3 ? 4 : group; }
 __host__ __device__ inline int rb_chunks(int group) { return (group + rb_heads(group) - 1) / rb_heads(group); }
@@ -1121,7 +1130,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
     for (int i = tid; i < kRbPairs * (DH / 4); i += 256) {
         const int pair = i % kRbPairs, c4 = i / kRbPairs;
         const int r = min(row0 + pair / hp, a.B - 1), h = h0 + min(pair % hp, nh - 1);
-        const float4 q = reinterpret_cast<const float4*>(a.q_rot + (int64_t(r) * a.Hq + h) * DH)[c4];
+        const float4 q = load_f4(a.q_rot + (int64_t(r) * a.Hq + h) * DH + 4 * c4);
         float* d = qs + 4 * c4 * kRbPairs + pair;
         d[0] = q.x, d[kRbPairs] = q.y, d[2 * kRbPairs] = q.z, d[3 * kRbPairs] = q.w;
     }
@@ -1135,7 +1144,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
             const float* k = kh + int64_t(c) * a.max_ctx;
             float4 v;
             if constexpr (decltype(whole)::value) {
-                __builtin_memcpy(&v, reinterpret_cast<const uint8_t*>(k) + uint32_t(4 * kl), 16);  // a uniform base and a 32-bit offset
+                v = load_f4(reinterpret_cast<const float*>(reinterpret_cast<const uint8_t*>(k) + uint32_t(4 * kl)));  // a uniform base and a 32-bit offset
             } else {  // the tile runs past the cache
                 const int last = int(a.max_ctx) - 1;
                 v = make_float4(k[min(kl, last)], k[min(kl + 1, last)], k[min(kl + 2, last)], k[min(kl + 3, last)]);
@@ -1173,7 +1182,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
             float* d = a.scores + int64_t(s.z) * a.max_ctx + kl - s.x;
             const float4 v = make_float4(a.score_scale * acc[p][0], a.score_scale * acc[p][1], a.score_scale * acc[p][2], a.score_scale * acc[p][3]);
             if (kl >= s.x && kl + 3 <= s.y) {
-                __builtin_memcpy(d, &v, 16);
+                store_f4(d, v);
             } else {
                 if (kl >= s.x && kl <= s.y) d[0] = v.x;
                 if (kl + 1 >= s.x && kl + 1 <= s.y) d[1] = v.y;
@@ -1458,7 +1467,7 @@ __global__ __launch_bounds__(kPrThreads) __attribute__((amdgpu_waves_per_eu(4, 4
 #pragma unroll
     for (int i = 0; i < PL; ++i) {
         const int pair = p0 + i, row = min(row0 + pair / hp, a.B - 1), h = h0 + min(pair % hp, nh - 1);
-        const float4 gate = *reinterpret_cast<const float4*>(a.proj + int64_t(row) * a.proj_stride + int64_t(h) * 2 * DH + DH + part * kAttnDim + cl);
+        const float4 gate = load_f4(a.proj + int64_t(row) * a.proj_stride + int64_t(h) * 2 * DH + DH + part * kAttnDim + cl);
         const float out[4] = {acc[i][0] * sigmoid_f32(gate.x), acc[i][1] * sigmoid_f32(gate.y), acc[i][2] * sigmoid_f32(gate.z), acc[i][3] * sigmoid_f32(gate.w)};
         float amax = 0.f;
 #pragma unroll
@@ -1469,7 +1478,7 @@ __global__ __launch_bounds__(kPrThreads) __attribute__((amdgpu_waves_per_eu(4, 4
         const float id = d != 0.f ? 1.f / d : 0.f;
         if (hi[i] >= 0) {
             const int64_t o = int64_t(row) * width + int64_t(h) * DH + part * kAttnDim + cl;
-            if (a.out_f32) *reinterpret_cast<float4*>(a.out_f32 + o) = make_float4(out[0], out[1], out[2], out[3]);
+            if (a.out_f32) store_f4(a.out_f32 + o, make_float4(out[0], out[1], out[2], out[3]));
             uint32_t pk = 0;
 #pragma unroll
             for (int e = 0; e < 4; ++e) pk |= uint32_t(uint8_t(int8_t(int(roundf(out[e] * id))))) << (8 * e);

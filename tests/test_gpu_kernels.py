@@ -790,6 +790,38 @@ def test_attn_prefill_pair_blocks_match_oracle(lib, M, p0, hq, hkv, max_ctx, win
     test_attn_prefill_rows_match_oracle(lib, M, p0, hq, hkv, max_ctx, window, dh)
 
 
+@pytest.mark.parametrize("M,p0,hq,hkv,dh", [(520, 0, 32, 8, 128), (9, 300, 8, 2, 128), (20, 30, 8, 4, 256)])
+def test_attn_prefill_takes_rows_at_any_float_address(lib, M, p0, hq, hkv, dh):
+    """An odd proj_stride and projections, rotated queries, scores and outputs
+    that start 4 bytes off a 16-byte boundary: the same bytes as from aligned
+    buffers."""
+    from hero_amd._lib import AttnDecodeArgs
+
+    rng = np.random.default_rng(M + dh)
+    qw, kw, max_ctx = hq * dh, hkv * dh, p0 + M + 1
+    width = 2 * qw + 2 * kw
+    proj = rng.standard_normal((M, width)).astype(np.float32)
+    kc = (rng.standard_normal((hkv, dh, max_ctx)) * 0.5).astype(np.float32)
+    vc = rng.standard_normal((max_ctx, kw)).astype(np.float32)
+    gamma = dev((1 + 0.1 * rng.standard_normal(dh)).astype(np.float32))
+    d_cs, d_pos = dev(oracle.rope_table(dh, 1e6, 32, max_ctx)), dev(np.arange(p0, p0 + M, dtype=np.int32))
+    res = []
+    for off in (0, 1):  # floats
+        rows = np.zeros((M, width + off), np.float32)
+        rows[:, :width] = proj
+        d_proj = dev(np.concatenate([np.zeros(off, np.float32), rows.ravel()]))
+        d_kc, d_vc = dev(kc), dev(vc)
+        d_sc, d_qr, out = (empty((n + off) * 4) for n in (M * hq * max_ctx, M * qw, M * qw))
+        act = empty(lib.hero_q8_0_act_bytes(M, qw))
+        at = lambda d: ptr(d) + 4 * off  # noqa: E731
+        a = AttnDecodeArgs(at(d_proj), width + off, 2 * qw, 2 * qw + kw, ptr(gamma), ptr(gamma), np.float32(1e-6), ptr(d_cs), ptr(d_kc), ptr(d_vc),
+                           max_ctx, ptr(d_pos), at(d_sc), at(d_qr), np.float32(0.09), 0, ptr(act), at(out), M, hq, hkv, dh)
+        check(lib.hero_attn_prefill(a, stream()))
+        res.append((host(out, np.uint32)[off:off + M * qw].copy(), host(act, np.uint8)[: lib.hero_q8_0_act_bytes(M, qw)].copy(), host(d_kc, np.uint32).copy()))
+    for aligned, shifted in zip(*res):
+        assert np.array_equal(aligned, shifted)
+
+
 @pytest.mark.parametrize("hq,window,page,dh", [(8, 0, 16, 128), (8, 50, 16, 128), (16, 0, 16, 128), (8, 0, 64, 128), (8, 50, 64, 128),
                                                 (8, 70, 64, 128), (16, 0, 64, 128), (8, 0, 64, 256), (8, 70, 64, 256), (16, 50, 64, 256)])
 def test_attn_paged_fp16_matches_oracle_over_fp16_kv(lib, hq, window, page, dh):
