@@ -822,6 +822,34 @@ def test_attn_prefill_takes_rows_at_any_float_address(lib, M, p0, hq, hkv, dh):
         assert np.array_equal(aligned, shifted)
 
 
+# blocks whose pairs are partly past the chunk or past the group's heads (groups
+# of 6: chunks of 4 and 2) form those pairs' sums from whatever the scratch holds
+@pytest.mark.parametrize("M,p0,hq,hkv,dh", [(203, 200, 12, 2, 128), (130, 90, 6, 1, 256), (530, 0, 40, 8, 128)])
+def test_attn_prefill_does_not_depend_on_scratch(lib, M, p0, hq, hkv, dh):
+    from hero_amd._lib import AttnDecodeArgs
+
+    rng = np.random.default_rng(M + dh)
+    qw, kw, max_ctx = hq * dh, hkv * dh, p0 + M + 2
+    stride = 2 * qw + 2 * kw
+    d_proj = dev(rng.standard_normal((M, stride)).astype(np.float32))
+    kc = (rng.standard_normal((hkv, dh, max_ctx)) * 0.5).astype(np.float32)
+    vc = rng.standard_normal((max_ctx, kw)).astype(np.float32)
+    gamma = dev((1 + 0.1 * rng.standard_normal(dh)).astype(np.float32))
+    d_cs, d_pos = dev(oracle.rope_table(dh, 1e6, 32, max_ctx)), dev(np.arange(p0, p0 + M, dtype=np.int32))
+    res = []
+    for fill in (0, 0xFF):  # zeros, NaNs
+        d_kc, d_vc = dev(kc), dev(vc)
+        d_sc, d_qr = dev(np.full(M * hq * max_ctx * 4, fill, np.uint8)), dev(np.full(M * qw * 4, fill, np.uint8))
+        out, act = empty(M * qw * 4), empty(lib.hero_q8_0_act_bytes(M, qw))
+        a = AttnDecodeArgs(ptr(d_proj), stride, 2 * qw, 2 * qw + kw, ptr(gamma), ptr(gamma), np.float32(1e-6), ptr(d_cs), ptr(d_kc), ptr(d_vc),
+                           max_ctx, ptr(d_pos), ptr(d_sc), ptr(d_qr), np.float32(0.09), 0, ptr(act), ptr(out), M, hq, hkv, dh)
+        check(lib.hero_attn_prefill(a, stream()))
+        res.append((host(out, np.uint32).copy(), host(act, np.uint8).copy()))
+    assert np.isfinite(res[0][0].view(np.float32)).all()
+    for zeros, nans in zip(*res):
+        assert np.array_equal(zeros, nans)
+
+
 @pytest.mark.parametrize("hq,window,page,dh", [(8, 0, 16, 128), (8, 50, 16, 128), (16, 0, 16, 128), (8, 0, 64, 128), (8, 50, 64, 128),
                                                 (8, 70, 64, 128), (16, 0, 64, 128), (8, 0, 64, 256), (8, 70, 64, 256), (16, 50, 64, 256)])
 def test_attn_paged_fp16_matches_oracle_over_fp16_kv(lib, hq, window, page, dh):
