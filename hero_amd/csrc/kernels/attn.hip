@@ -1503,11 +1503,28 @@ static int64_t pv_row_blocks(const AttnDecodeArgs& a, int PL) {
     return int64_t(a.Hkv) * rb_chunks(group) * (a.Dh / kAttnDim) * ((a.B + R - 1) / R);
 }
 
-// Which prefill chunks run in pair blocks: all but short ones under a sliding
-// window, where the per-row kernels' many workgroups are faster while the pair
-// blocks leave half the compute units without one (16 rows, window 512: 27 us
-// against 32; 128 rows 72 against 38).
-static bool attn_prefill_in_blocks(const AttnDecodeArgs& a) { return a.window == 0 || 2 * pv_row_blocks(a, 2) >= device_cus(); }
+// Which prefill chunks run in pair blocks; the others take the per-row kernels,
+// whose many workgroups each walk one row's keys, while a pair block walks them
+// once for its rows, however few.
+static bool attn_prefill_in_blocks(const AttnDecodeArgs& a) {
+    // Sliding windows: while the pair blocks leave half the compute units without
+    // one the per-row kernels are faster (16 rows, window 512: 27 us against 32;
+    // 128 rows 72 against 38).
+    if (a.window > 0) return 2 * pv_row_blocks(a, 2) >= device_cus();
+    // Full visibility, in microseconds: the per-row kernels cost per row (of 32
+    // heads of 128) and per row and key, the blocks' walk per key, and 8 more to
+    // begin with. Fitted over 1 to 128 rows after 0 to 8191, 8 to 64 query heads.
+    // 32 heads of 128, per-row kernels and pair blocks: 16 rows alone 26 / 26, 64
+    // 59 / 29; after 1023: 8 rows 34 / 112, 64 rows 129 / 133; after 8191: 1 row 84
+    // / 700, 64 rows 606 / 850.
+    // How far the sequence is the host does not know: taken as the rows alone, the
+    // least it can be, where a prompt's first chunk must not lose. Caches that are
+    // no multiple of 4 long are taken as full: the per-row kernels always ran
+    // these chunks, and late ones would lose most.
+    const double ctx = a.max_ctx % 4 == 0 ? a.B : double(a.max_ctx);
+    const double rows = double(a.B) * double(a.Hq) * a.Dh / 4096 * (0.5 + 0.0009 * ctx), walk = 8 + 0.085 * ctx;
+    return rows > walk;
+}
 
 template <int DH>
 static void attn_prefill_rows(const AttnDecodeArgs& a, hipStream_t s) {

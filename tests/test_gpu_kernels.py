@@ -719,11 +719,11 @@ def test_attn_decode_long_context_matches_oracle(lib, B, hq, hkv, pos, window, d
 
 # a prefill chunk: M consecutive tokens of one sequence after p0 cached rows,
 # all sharing cache 0 (the reference appends the whole batch, then reduces
-# each row over its visible rows). max_ctx % 4 == 0 with no window takes the
-# register softmax and the row-block weighted sum (blocks of 8 rows: 37 and
-# 603 rows leave a partial last block; group 6 makes head chunks of 4 and 2;
-# p0 = 4100 gives rows of more than 4096 keys, the chunked softmax);
-# max_ctx % 4 != 0 and the window take the per-row kernels.
+# each row over its visible rows). Many rows run in pair blocks (603 rows leave
+# a partial last block, 300 of 256-wide heads); the others and the window run
+# the per-row kernels (group 6 makes head chunks of 4 and 2; p0 = 4100 gives
+# rows of more than 4096 keys; max_ctx % 4 != 0 the softmax without 16-byte
+# rows). The tests below hold the edges of either form.
 @pytest.mark.parametrize("M,p0,hq,hkv,max_ctx,window,dh", [(37, 0, 8, 2, 40, 0, 128), (603, 70, 32, 8, 676, 0, 128), (20, 33, 6, 1, 56, 0, 128),
                                                            (64, 4100, 8, 2, 4168, 0, 128), (10, 5, 4, 1, 17, 0, 128), (24, 9, 8, 2, 36, 7, 128),
                                                            (300, 40, 16, 4, 344, 0, 256), (12, 3, 8, 2, 17, 0, 256)])
@@ -783,14 +783,41 @@ def test_attn_prefill_rows_match_oracle(lib, M, p0, hq, hkv, max_ctx, window, dh
 # score tile; 530 rows of 256-wide heads (four pairs a lane); groups of 1, 2
 # and 5 heads; a window whose scale of 1 spreads the scores so far that weights
 # underflow (the division beside the fast quotient), over a row stride that is
-# no multiple of 4; bit for bit, as the test above
+# no multiple of 4; bit for bit, as the test above (few rows of few heads run
+# per row: the shapes of groups 1, 2 and 5 come again with enough rows)
 @pytest.mark.parametrize("M,p0,hq,hkv,max_ctx,window,dh", [(513, 0, 24, 8, 513, 0, 128), (530, 3, 32, 8, 535, 0, 256), (20, 5, 4, 4, 32, 0, 128), (21, 300, 8, 4, 323, 0, 128),
                                                            (33, 7, 10, 2, 42, 0, 256), (130, 60, 32, 8, 191, 50, 128), (1, 30, 8, 2, 40, 0, 128)])
 def test_attn_prefill_pair_blocks_match_oracle(lib, M, p0, hq, hkv, max_ctx, window, dh):
     test_attn_prefill_rows_match_oracle(lib, M, p0, hq, hkv, max_ctx, window, dh)
 
 
-@pytest.mark.parametrize("M,p0,hq,hkv,dh", [(520, 0, 32, 8, 128), (9, 300, 8, 2, 128), (20, 30, 8, 4, 256)])
+# groups of 1, 2, 4, 5 and 6 heads, ragged blocks, rows of more than 4096 keys and a
+# cache no multiple of 4 long, in pair blocks (rows x heads x Dh / 4096 x (0.5 +
+# 0.0009 n) > 8 + 0.085 n, n the rows or, for such a cache, its length)
+@pytest.mark.parametrize("M,p0,hq,hkv,max_ctx,dh", [(410, 5, 4, 4, 416, 128), (203, 11, 8, 4, 216, 128), (67, 7, 10, 2, 74, 256), (301, 3, 6, 1, 305, 128),
+                                                    (61, 4100, 32, 8, 4164, 128), (130, 60, 6, 1, 192, 256)])
+def test_attn_prefill_pair_blocks_of_every_group_match_oracle(lib, M, p0, hq, hkv, max_ctx, dh):
+    test_attn_prefill_rows_match_oracle(lib, M, p0, hq, hkv, max_ctx, 0, dh)
+
+
+# few rows, on the per-row kernels: one and two rows (the fused softmax and sum up
+# to 4096 positions), up to four (the per-head pipelines beyond), more (the
+# many-sequence form), both head widths, caches no multiple of 4 long
+@pytest.mark.parametrize("M,p0,hq,hkv,max_ctx,dh", [(1, 50, 32, 8, 64, 128), (2, 300, 32, 8, 304, 128), (2, 40, 32, 8, 43, 128), (1, 4100, 32, 8, 4104, 128),
+                                                    (4, 4100, 32, 8, 4104, 128), (9, 50, 32, 8, 60, 128), (2, 60, 8, 2, 64, 256), (1, 4100, 8, 2, 4104, 256),
+                                                    (9, 30, 8, 2, 41, 256)])
+def test_attn_prefill_few_rows_match_oracle(lib, M, p0, hq, hkv, max_ctx, dh):
+    test_attn_prefill_rows_match_oracle(lib, M, p0, hq, hkv, max_ctx, 0, dh)
+
+
+# windows: 256-wide heads in pair blocks (64 rows of 8 K/V heads) and per row, a
+# short chunk over a cache no multiple of 4 long
+@pytest.mark.parametrize("M,p0,hq,hkv,max_ctx,window,dh", [(64, 40, 32, 8, 104, 50, 256), (24, 40, 8, 2, 64, 30, 256), (9, 20, 8, 2, 31, 12, 128), (2, 90, 8, 2, 92, 40, 128)])
+def test_attn_prefill_windows_match_oracle(lib, M, p0, hq, hkv, max_ctx, window, dh):
+    test_attn_prefill_rows_match_oracle(lib, M, p0, hq, hkv, max_ctx, window, dh)
+
+
+@pytest.mark.parametrize("M,p0,hq,hkv,dh", [(520, 0, 32, 8, 128), (64, 300, 32, 8, 128), (70, 30, 8, 4, 256)])
 def test_attn_prefill_takes_rows_at_any_float_address(lib, M, p0, hq, hkv, dh):
     """An odd proj_stride and projections, rotated queries, scores and outputs
     that start 4 bytes off a 16-byte boundary: the same bytes as from aligned
