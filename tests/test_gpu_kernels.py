@@ -1064,12 +1064,12 @@ def test_kquant_gemm_many_rows_matches_oracle_bitwise(lib, wtype, m, n, k):
     assert bad.size == 0, f"{bad.size} outputs differ, first {bad[:5]}"
 
 
-# the matrix-core form: edges of its 32- and 64-row tiles in
-# both directions, one super-block per row (256 rows per packed tile), rows of
-# 256 super-blocks (one row per packed tile), and grids that take the large
-# tile (more than two rounds of small ones). Every intermediate is an exact
-# integer or one correctly rounded fp32 operation in the reference's order, so
-# the outputs are equal bit for bit.
+# the matrix-core form: edges of its 32-row tiles in both directions, one
+# super-block per row (256 rows per packed tile), rows of 256 super-blocks (one
+# row per packed tile), the 64-row tile (130 rows; more in the next test), and
+# 70 x 8193, K 256, which the lane-per-block form takes. Every intermediate is an
+# exact integer or one correctly rounded fp32 operation in the reference's
+# order, so the outputs are equal bit for bit.
 @pytest.mark.parametrize("wtype", [12, 14])
 @pytest.mark.parametrize("m,n,k", [(9, 1, 256), (31, 33, 256), (32, 32, 512), (33, 31, 768), (65, 97, 1024), (32, 450, 65536), (130, 4100, 512), (70, 8193, 256)])
 def test_kquant_matrix_core_form_matches_oracle_bitwise(lib, wtype, m, n, k):
@@ -1080,6 +1080,36 @@ def test_kquant_matrix_core_form_matches_oracle_bitwise(lib, wtype, m, n, k):
     x[m - 1] = 0.0
     _, y = kquant_dev(lib, wtype, w, x, n, k)
     expect = oracle.matmul_kquant(wtype, w, n, k, x)
+    bad = np.flatnonzero(bits(y).ravel() != bits(expect).ravel())
+    assert bad.size == 0, f"{bad.size} outputs differ, first {bad[:5]}: {y.ravel()[bad[:3]]} vs {expect.ravel()[bad[:3]]}"
+
+
+def kquant_plan(lib, wtype, m, n, k):
+    import ctypes
+
+    kernel = ctypes.c_int32()
+    check(lib.hero_kquant_gemm_plan(wtype, m, n, k, ctypes.byref(kernel)))
+    return kernel.value
+
+
+# the 64-row tile with 1, 2, 3, 11 and 16 super-blocks a row (the third one writes
+# the first shared-memory buffer again) and the 32-row one with 11 and 16, ragged
+# both ways; the form that each shape takes is part of the test. The second row's
+# largest value is 5e-37: its scale (1 / 127 of that) and the products of its
+# scale with the weights' are subnormal.
+@pytest.mark.parametrize("wtype", [12, 14])
+@pytest.mark.parametrize("m,n,k,form", [(129, 4100, 256, 64), (130, 4100, 512, 64), (129, 4163, 768, 64), (97, 4100, 2816, 64), (70, 6000, 4096, 64),
+                                        (66, 5000, 2816, 32), (19, 4099, 4096, 32), (70, 8193, 256, 1), (2, 300, 4096, 1)])
+def test_kquant_products_of_every_form_match_oracle_bitwise(lib, wtype, m, n, k, form):
+    assert kquant_plan(lib, wtype, m, n, k) == form
+    rng = np.random.default_rng(wtype * 101 + m + n + k)
+    w = kquant_weights(rng, wtype, n, k)
+    x = (rng.standard_normal((m, k)) * np.exp(rng.uniform(-20, 20, (m, 1)))).astype(np.float32)
+    x[0] = np.where(rng.random(k) < 0.5, 1.0, -1.0)
+    x[1] *= 5e-37 / np.abs(x[1]).reshape(-1, 256).max(1).repeat(256)
+    _, y = kquant_dev(lib, wtype, w, x, n, k)
+    expect = oracle.matmul_kquant(wtype, w, n, k, x)
+    assert np.any(expect[1] != 0)
     bad = np.flatnonzero(bits(y).ravel() != bits(expect).ravel())
     assert bad.size == 0, f"{bad.size} outputs differ, first {bad[:5]}: {y.ravel()[bad[:3]]} vs {expect.ravel()[bad[:3]]}"
 
@@ -1123,13 +1153,14 @@ def test_q5_K_gemm_matches_oracle_bitwise(lib, m, n, k):
     assert bad.size == 0, f"{bad.size} outputs differ, first {bad[:5]}"
 
 
-# the outer-product form: edges of its 4- and 16-row tiles and 64-row weight
-# tiles, fewer super-blocks than waves, more than a round of them; the tiny
+# the outer-product form: edges of its 4- and 16-row tiles (16 from 250 rows on)
+# and 64-row weight tiles, fewer super-blocks than waves, more than a round of them; the tiny
 # scales make products and sums subnormal. Products and sums are each rounded
 # once, in the reference's order: equal bit for bit.
 @pytest.mark.parametrize("m,n,k", [(2, 1, 256), (3, 65, 256), (5, 64, 1024), (10, 4097, 2304), (70, 800, 5120), (14, 2050, 8192), (250, 1020, 2304), (497, 511, 1280)])
 @pytest.mark.parametrize("scale", [1.0, 1e-36])
 def test_q5_K_outer_product_form_matches_oracle_bitwise(lib, m, n, k, scale):
+    assert kquant_plan(lib, 13, m, n, k) == (16 if m >= 250 else 4)
     rng = np.random.default_rng(m * 1009 + n * 31 + k)
     w = q5k_weights(rng, n, k)
     x = (rng.standard_normal((m, k)) * scale).astype(np.float32)
