@@ -597,7 +597,7 @@ __global__ __launch_bounds__(kPvThreads) void attn_pv_kernel(AttnDecodeArgs a) {
         const int64_t width = int64_t(a.Hq) * kAttnDim;
         const int64_t idx = int64_t(h) * kAttnDim + ch;
         if (a.out_f32) a.out_f32[int64_t(b) * width + idx] = out;
-        float amax = fabsf(out);
+        float amax = fmaxf(0.f, fabsf(out));  // a block of NaNs: 0, as the reference's running maximum
         for (int off = 16; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 32));
         const float d = amax / 127.f;
         const float id = d != 0.f ? 1.f / d : 0.f;
@@ -827,7 +827,7 @@ __global__ __launch_bounds__(kSpvThreads) void attn_softmax_pv_kernel(AttnDecode
         const int64_t width = int64_t(a.Hq) * DH;
         const int64_t idx = int64_t(h) * DH + ch;
         if (a.out_f32) a.out_f32[int64_t(b) * width + idx] = out;
-        float amax = fabsf(out);
+        float amax = fmaxf(0.f, fabsf(out));  // a block of NaNs: 0, as the reference's running maximum
         for (int off = 16; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 32));
         const float d = amax / 127.f;
         const float id = d != 0.f ? 1.f / d : 0.f;
@@ -971,7 +971,7 @@ __global__ __launch_bounds__(kPvbThreads) void attn_pv_batch_kernel(AttnDecodeAr
         const int64_t width = int64_t(a.Hq) * DH;
         const int64_t idx = int64_t(h) * DH + ch;
         if (a.out_f32) a.out_f32[int64_t(b) * width + idx] = out;
-        float amax = fabsf(out);
+        float amax = fmaxf(0.f, fabsf(out));  // a block of NaNs: 0, as the reference's running maximum
         for (int off = 16; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 32));
         const float d = amax / 127.f;
         const float id = d != 0.f ? 1.f / d : 0.f;

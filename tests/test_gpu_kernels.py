@@ -877,6 +877,33 @@ def test_attn_prefill_does_not_depend_on_scratch(lib, M, p0, hq, hkv, dh):
         assert np.array_equal(zeros, nans)
 
 
+# a sequence with a NaN value row: every output that sees it is NaN, and a block of
+# 32 NaNs gets the reference's scale (its running maximum skips NaNs: 0) from
+# every form, so that the form a chunk takes does not show
+@pytest.mark.parametrize("M,p0,hq,hkv,max_ctx,window,dh", [(1, 40, 32, 8, 64, 0, 128), (1, 40, 32, 8, 63, 0, 128), (4, 40, 32, 8, 63, 0, 128), (9, 40, 32, 8, 64, 0, 128),
+                                                           (3, 40, 8, 2, 64, 20, 128), (9, 40, 8, 2, 64, 0, 256), (64, 40, 32, 8, 104, 0, 128), (130, 40, 32, 8, 172, 100, 128)])
+def test_attn_prefill_nan_blocks_have_the_reference_scale(lib, M, p0, hq, hkv, max_ctx, window, dh):
+    from hero_amd._lib import AttnDecodeArgs
+
+    rng = np.random.default_rng(M + p0)
+    qw, kw = hq * dh, hkv * dh
+    stride = 2 * qw + 2 * kw
+    proj = rng.standard_normal((M, stride)).astype(np.float32)
+    proj[0, 2 * qw + kw: 2 * qw + kw + dh] = np.nan  # the first new token's values of K/V head 0
+    d_kc, d_vc = dev((rng.standard_normal((hkv, dh, max_ctx)) * 0.5).astype(np.float32)), dev(rng.standard_normal((max_ctx, kw)).astype(np.float32))
+    gamma = dev((1 + 0.1 * rng.standard_normal(dh)).astype(np.float32))
+    d_proj, d_cs, d_pos = dev(proj), dev(oracle.rope_table(dh, 1e6, 32, max_ctx)), dev(np.arange(p0, p0 + M, dtype=np.int32))
+    d_sc, d_qr, out, act = empty(M * hq * max_ctx * 4), empty(M * qw * 4), empty(M * qw * 4), empty(lib.hero_q8_0_act_bytes(M, qw))
+    a = AttnDecodeArgs(ptr(d_proj), stride, 2 * qw, 2 * qw + kw, ptr(gamma), ptr(gamma), np.float32(1e-6), ptr(d_cs), ptr(d_kc), ptr(d_vc),
+                       max_ctx, ptr(d_pos), ptr(d_sc), ptr(d_qr), np.float32(0.09), window, ptr(act), ptr(out), M, hq, hkv, dh)
+    check(lib.hero_attn_prefill(a, stream()))
+    got = host(out, np.float32, (M, qw))
+    assert np.isnan(got[0, : hq // hkv * dh]).all() and not np.isnan(got[:, hq // hkv * dh:]).any()
+    blocks = act_to_blocks(host(act, np.uint8), M, qw)
+    for b in range(M):
+        assert blocks[b].tobytes() == oracle.quantize_row_q8_0(got[b]).tobytes(), f"row {b}"
+
+
 @pytest.mark.parametrize("hq,window,page,dh", [(8, 0, 16, 128), (8, 50, 16, 128), (16, 0, 16, 128), (8, 0, 64, 128), (8, 50, 64, 128),
                                                 (8, 70, 64, 128), (16, 0, 64, 128), (8, 0, 64, 256), (8, 70, 64, 256), (16, 50, 64, 256)])
 def test_attn_paged_fp16_matches_oracle_over_fp16_kv(lib, hq, window, page, dh):
