@@ -7,8 +7,8 @@
 //
 // Four stages, each keeping the reference's fp32 operation order (the fused
 // and tiled forms further down -- score tiles with the prep folded in, the
-// softmax and weighted sum in one kernel, the register softmax, the row-block
-// weighted sum of prefill -- compute the same values):
+// softmax and weighted sum in one kernel, the register softmax, the pair blocks
+// of prefill -- compute the same values):
 //  1. prep    one workgroup per (sequence, query head), a lane per channel:
 //             split of the packed [q | gate] pair, q RMSNorm + RoPE; the first
 //             query head of each K/V group also normalises and rotates k and

@@ -567,10 +567,10 @@ __global__ __launch_bounds__(kGdnDim) void gdn_norm_gate_kernel(const float* __r
 //  scan  the delta rule over the tokens in order, 8 workgroups per value
 //        head, the state in registers for the whole chunk (below);
 //  out   (token, head) in parallel: head RMSNorm, SiLU(z) gate, quantize.
-// The scan's critical path per token is one 128-term chain: token t's output
-// chain and token t+1's decay and prediction chain read the same updated
-// column, so they run side by side. Every value is computed by the same
-// operations in the same order as in gdn_decode_kernel.
+// The scan's critical path per token is one 128-term chain, the prediction, which
+// has waves of its own; the outputs' chains run beside it, a tile behind. Every
+// value is computed by the same operations in the same order as in
+// gdn_decode_kernel.
 
 __device__ __forceinline__ GdnPrefillWork gdn_work(void* ws, int64_t T, int Hk, int Hv) {
     GdnPrefillWork w;
