@@ -793,9 +793,10 @@ def test_attn_prefill_pair_blocks_match_oracle(lib, M, p0, hq, hkv, max_ctx, win
 
 # groups of 1, 2, 4, 5 and 6 heads, ragged blocks, rows of more than 4096 keys and a
 # cache no multiple of 4 long, in pair blocks (rows x heads x Dh / 4096 x (0.5 +
-# 0.0009 n) > 8 + 0.085 n, n the rows or, for such a cache, its length)
+# 0.0009 n) > 8 + 0.085 n, n the rows or, for such a cache, its length); 500 rows
+# of 16 K/V heads give each lane of the 128-wide weighted sum four pairs
 @pytest.mark.parametrize("M,p0,hq,hkv,max_ctx,dh", [(410, 5, 4, 4, 416, 128), (203, 11, 8, 4, 216, 128), (67, 7, 10, 2, 74, 256), (301, 3, 6, 1, 305, 128),
-                                                    (61, 4100, 32, 8, 4164, 128), (130, 60, 6, 1, 192, 256)])
+                                                    (61, 4100, 32, 8, 4164, 128), (130, 60, 6, 1, 192, 256), (500, 9, 64, 16, 512, 128)])
 def test_attn_prefill_pair_blocks_of_every_group_match_oracle(lib, M, p0, hq, hkv, max_ctx, dh):
     test_attn_prefill_rows_match_oracle(lib, M, p0, hq, hkv, max_ctx, 0, dh)
 
